@@ -149,7 +149,7 @@ def main():
     ap.add_argument("--cg-warm", type=int, choices=[0, 1], default=1,
                     help="start a step's first solve from the previous step's solution (0 = from zero)")
     ap.add_argument("--cg-wide", type=int, choices=[0, 1], default=1,
-                    help="exact tiled band-Cholesky preconditioner for banded systems above 1,024 equations")
+                    help="exact tiled sparse factor as preconditioner under the static integrators")
     args = ap.parse_args()
     if args.gpus != 1:
         print(json.dumps({"error": "this build runs on one GPU; --gpus must be 1"}))

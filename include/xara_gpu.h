@@ -75,13 +75,14 @@ typedef struct xg_counters {
   double    time_tangent_ms;
   double    time_unbalance_ms;
   double    time_solve_ms;
-  long long band_bw;          /* half bandwidth of the band-Cholesky
-                                 preconditioner, -1 when it is not used    */
-  long long band_fallbacks;   /* matrices whose tiled band factor met a pivot
+  long long band_bw;          /* half bandwidth of the matrix in the band
+                                 order when an exact factor (band or tiled)
+                                 preconditions the PCG, -1 otherwise       */
+  long long band_fallbacks;   /* matrices whose exact factor met a pivot
                                  that is not positive and were solved with
                                  block Jacobi instead                      */
   long long band_reuses;      /* assembled matrices equal bit for bit to the
-                                 last one factored, whose band factor was
+                                 last one factored, whose factor was
                                  kept instead of formed again              */
 } xg_counters;
 
@@ -202,11 +203,11 @@ int  xg_spmv_config(xg_domain* d, int format, int lanes);
                           preconditioned solves; the default; the stop test
                           stays |r| <= rtol |b|)                               */
 #define XG_CG_WIDE  16 /* with XG_CG_SMALL, under LoadControl and
-                          DisplacementControl: systems of more than 1,024
-                          equations whose half bandwidth in the band order is
-                          at most 1,024 are preconditioned by their exact band
-                          Cholesky factor, formed in 64 x 64 tiles (one or two
-                          PCG iterations per solve); on by default           */
+                          DisplacementControl: systems of 385 to 262,144
+                          equations are preconditioned by their exact tiled
+                          sparse factor in nested-dissection order (one or
+                          two PCG iterations per solve) where it fits in
+                          2 x 1 GiB; on by default                          */
 int  xg_cg_config(xg_domain* d, int chunk, int flags);
 /* `numberer RCM|Plain`                                                       */
 int  xg_numberer(xg_domain* d, int kind);
@@ -271,7 +272,7 @@ int  xg_solve(xg_domain* d, const double* B, double* X);
    xg_solve; every PCG work buffer (staging of B and X, the six iteration
    vectors, the block-Jacobi inverses or the one-workgroup band factor,
    partial sums, scalars) comes from a fixed 128 MiB device array per GPU,
-   looked up at xg_create; the tiled band factor (XG_CG_WIDE) uses the
+   looked up at xg_create; the tiled factor (XG_CG_WIDE) uses the
    domain's own buffers, allocated at xg_setup; the kernels are launched
    one by one (no graph).  A system whose buffers do not fit (about 1.1 M
    equations with nodal 3x3 blocks) is XG_ERR_ARG.  Calls that overlap on

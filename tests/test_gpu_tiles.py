@@ -1,0 +1,107 @@
+"""GPU parity of the tiled sparse factorisation (xg_tiles.hip) against the
+CPU oracle's direct solve, at the edges of its sizes: the fewest equations
+it takes, columns of 1 to 64 equations, one to many levels, DOFs fixed inside
+the model, 1 to many sources per update; single solves, the allocation-free
+solve bit for bit, and the paired solves of DisplacementControl."""
+import numpy as np
+import pytest
+
+from tests import _oracle
+from xara_amd import _lib, meshes
+from xara_amd.model import Model
+
+pytestmark = pytest.mark.gpu
+EPS = np.finfo(float).eps
+
+
+def relerr(a, b):
+    return float(np.max(np.abs(a - b)) / np.max(np.abs(b)))
+
+
+def build(case, m):
+    kind, *size = case
+    if kind == "quad":
+        mesh = meshes.quad_strip(*size)
+        mesh["crds"] = mesh["crds"] + np.random.default_rng(1).uniform(-0.02, 0.02, mesh["crds"].shape)
+        meshes.build_quad_strip(m, mesh)
+        m.fix(mesh["tip"] - 2, 0, 1)
+        return mesh["tip"], 2, 1e-3, np.random.default_rng(2).normal(0, 1e-3, mesh["crds"].shape)
+    if kind == "brick":
+        mesh = meshes.brick_cube(size[0])
+        meshes.build_brick_cube(m, mesh)
+        return int(mesh["load_tags"][0]), 3, -1e-3, np.random.default_rng(2).normal(0, 1e-4, mesh["crds"].shape)
+    fr = meshes.rc_frame_3d(*size)
+    meshes.build_rc_frame_3d(m, fr)
+    U = np.random.default_rng(2).normal(0, 1e-2, (len(fr["crds"]), 6))
+    U[:, 3:] *= 1e-4
+    return fr["roof"], 1, 2.0, U
+
+
+CASES = [("quad", 14, 13), ("quad", 15, 13), ("quad", 5, 40), ("quad", 97, 1), ("quad", 61, 17), ("brick", 5),
+         ("brick", 9), ("frame", 3, 2, 6), ("frame", 7, 1, 11)]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "_".join(map(str, c)))
+def test_tiled_solve_matches_oracle(case):
+    print(f"case: tiled solve {case}", flush=True)
+    ndm, ndf = {"quad": (2, 2), "brick": (3, 3), "frame": (3, 6)}[case[0]]
+    g, o = Model(ndm, ndf), _oracle.oracle_model(ndm, ndf)
+    for m in (g, o):
+        node, dof, incr, U = build(case, m)
+        if case[0] == "quad":
+            m.load(node, 0.0, 1.0)
+        m.system("GpuBlockPCG", 1e-13, 1000)
+        m.setup()
+        m.set_trial_disp(U)
+        m.update()
+        m.form_tangent(values=False)
+    # residual: the iteration's own stop test (1e-13 |b|) and the rounding of
+    # the product it is formed with, eps sum |A| |x| per row; solutions to
+    # the condition number times the rounding, below the parity bar of 1e-9
+    rp, ci = o.csr_pattern()
+    absA = np.abs(o.form_tangent())
+    row = np.repeat(np.arange(o.neq), np.diff(rp))
+    for seed in range(3):
+        B = np.random.default_rng(seed).normal(size=g.neq)
+        c0 = g.counters()
+        X = g.solve(B)
+        c1 = g.counters()
+        assert c1["band_bw"] > 0 and c1["cg_iters"] - c0["cg_iters"] <= 2
+        noise = np.bincount(row, absA * np.abs(X)[ci], o.neq)
+        assert np.linalg.norm(o.spmv(X) - B) <= 1e-13 * np.linalg.norm(B) + 4 * EPS * np.linalg.norm(noise)
+        assert relerr(X, o.solve(B)) <= 1e-9
+        Xn = np.zeros_like(X)
+        assert g._b.solve_noalloc(g._h, B.ctypes.data_as(_lib.P_D), Xn.ctypes.data_as(_lib.P_D)) == 0
+        assert np.array_equal(X, Xn)
+    for m in (g, o):
+        m.revert_to_start()
+        m.test("NormUnbalance", 1e-6 if case[0] != "frame" else 1e-3, 30)
+        m.integrator("DisplacementControl", node, dof, incr)
+        assert m.analyze(3) == 0
+    assert relerr(g.trial_disp(), o.trial_disp()) <= 1e-9
+    assert abs(g.load_factor - o.load_factor) <= 1e-9 * abs(o.load_factor)
+    for m in (g, o):
+        m.close()
+
+
+def test_equation_limit():
+    """384 equations (16 x 12 x 2) stay with the solves that take fewer, 385
+    (one more DOF freed at the clamped end) are factored; the same solutions
+    with and without."""
+    for free in (0, 1):
+        m = Model(2, 2)
+        mesh = meshes.quad_strip(16, 11)
+        if free:
+            mesh["fixed_nodes"] = mesh["fixed_nodes"][1:]
+        meshes.build_quad_strip(m, mesh)
+        if free:
+            m.fix(1, 1, 0)
+        m.cg_config(wide=True)
+        m.setup()
+        assert m.neq == 384 + free
+        m.form_tangent(values=False)
+        B = np.ones(m.neq)
+        X = m.solve(B)
+        m.cg_config(wide=False)
+        assert relerr(X, m.solve(B)) <= 1e-9
+        m.close()

@@ -13,6 +13,7 @@
 #include "xg_j2.h"
 #include "xg_kernels.h"
 #include "xg_sym_layout.h"
+#include "xg_tileplan.h"
 
 namespace xg {
 
@@ -214,6 +215,7 @@ struct J2Group : Group {
 // ---------------------------------------------------------------------------
 Domain::~Domain() {
   cg_graph_clear();
+  if (tl_read) (void)hipHostFree(tl_read);
   if (ev0) (void)hipEventDestroy(ev0);
   if (ev1) (void)hipEventDestroy(ev1);
   groups.clear();
@@ -823,7 +825,7 @@ void Domain::form_tangent() {
 
 Domain::CgBufs Domain::cg_bufs() {
   return CgBufs{r0.p, r1.p, z.p, p.p, p2.p, q.p, part.p, binv.p, pcbad.p, scal.p, band_A.p, band_L.p, band_Lr.p,
-                sw_b.p, sw_x.p, binv_s.p, true};
+                sw_b.p, sw_x.p, binv_s.p};
 }
 
 // The preconditioner of the current matrix into w: the band-Cholesky factor
@@ -831,10 +833,10 @@ Domain::CgBufs Domain::cg_bufs() {
 // inverses.  Formed once per matrix and buffer set.
 void Domain::precond_setup(const CgBufs& w) {
   const bool band = band_active();
-  const bool wide = !band && !small_path() && w.wide && wide_active();
+  const bool wide = wide_active();
   const bool sweep = !band && !wide && !small_path() && sweep_active(w);
   const void* key = band   ? (const void*)w.bandL
-                    : wide ? (const void*)wb_L.p
+                    : wide ? (const void*)tl_G.p
                     : sweep ? (const void*)w.binvs
                             : (const void*)w.binv;
   if (pc_done == key) return;
@@ -861,7 +863,7 @@ void Domain::precond_setup(const CgBufs& w) {
   }
   XG_HIP(hipMemsetAsync(w.pcbad, 0, sizeof(int), stream));
   if (wide) {
-    wb_factor(w.pcbad);
+    tiles_form(w.pcbad);
   } else if (band) {
     band_factor(stream, num.neq, band_bw, rowptr.p, colind.p, vals.p, band_pinv.p, w.bandA, w.bandL, w.bandLr,
                 w.pcbad);
@@ -874,12 +876,11 @@ void Domain::precond_setup(const CgBufs& w) {
   pc_done = key;
 }
 
-// The wide-band factor of the current matrix; the launch sequence (one
-// per tile column) replayed from a captured graph when cg_graph_on.
-void Domain::wb_factor(int* bad) {
-  const int n = num.neq;
+// The tiled factor of the current matrix; its launches (two per level)
+// replayed from a captured graph when cg_graph_on.
+void Domain::tiles_form(int* bad) {
   auto run = [&] {
-    wband_factor(stream, n, wb_bw, rowptr.p, colind.p, vals.p, band_pinv.p, wb_L.p, wb_D.p, bad);
+    tiles_factor(stream, num.neq, tl_view, tl_host, rowptr.p, colind.p, vals.p, tl_A.p, tl_G.p, bad);
   };
   // plain launches when graphs are off or the flag is not the domain's own
   // (the allocation-free solve: the captured graph is left as it is)
@@ -887,111 +888,139 @@ void Domain::wb_factor(int* bad) {
     run();
     return;
   }
-  if (!wb_fe) capture_graph(stream, run, &wb_fg, &wb_fe);
-  XG_HIP(hipGraphLaunch(wb_fe, stream));
+  if (!tl_fe) capture_graph(stream, run, &tl_fg, &tl_fe);
+  XG_HIP(hipGraphLaunch(tl_fe, stream));
 }
 
-// z = M^-1 r for k = 1 or 2 right-hand sides, M the wide-band factor.
-void Domain::wb_apply(int k, const double* const* r, double* const* z, bool graphs) {
-  const int n = num.neq;
-  const size_t np = (size_t)wband_padded(n);
-  double* Yb = wb_Y.p;
-  double* Yo = Yb + 2 * np;
-  double* Xo = Yo + 2 * np;
-  for (int s = 0; s < k; s++) wband_perm_in(stream, n, wb_bw, band_pinv.p, r[s], Yb + s * np);
-  auto run = [&] { wband_sweeps(stream, n, wb_bw, k, wb_L.p, wb_D.p, Yb, Yo, Xo); };
+// z = M^-1 r for k = 1 or 2 right-hand sides, M the tiled factor.
+void Domain::tiles_apply(int k, const double* const* r, double* const* z, bool graphs) {
+  const size_t np = (size_t)kTile * tl_view.nt;
+  for (int s = 0; s < k; s++) tiles_in(stream, tl_view, r[s], tl_Y.p + s * np);
+  auto run = [&] { tiles_sweeps(stream, tl_view, tl_host, k, tl_G.p, tl_Y.p, tl_X.p); };
   if (graphs) {
-    if (!wb_se[k - 1]) capture_graph(stream, run, &wb_sg[k - 1], &wb_se[k - 1]);
-    XG_HIP(hipGraphLaunch(wb_se[k - 1], stream));
+    if (!tl_se[k - 1]) capture_graph(stream, run, &tl_sg[k - 1], &tl_se[k - 1]);
+    XG_HIP(hipGraphLaunch(tl_se[k - 1], stream));
   } else {
     run();
   }
-  for (int s = 0; s < k; s++) wband_perm_out(stream, n, band_pinv.p, Xo + s * np, z[s]);
+  for (int s = 0; s < k; s++) tiles_out(stream, num.neq, tl_view, tl_X.p + s * np, z[s]);
 }
 
-// PCG preconditioned by the exact wide-band factor, for R = 1 or 2
-// right-hand sides side by side (the preconditioner applied to both in one
-// set of sweeps): from x = 0, stopping at |r| <= rtol |b| like the other
-// paths.  The factor makes the first iterate the direct solution up to
-// rounding, so a solve takes one or two iterations.
+// PCG preconditioned by the exact tiled factor, for R = 1 or 2 right-hand
+// sides side by side (the preconditioner applied to both in one set of
+// sweeps): from x = 0, or from the guess in x (bit s of warm), stopping at
+// |r| <= rtol |b| like the other paths.  The factor makes the first iterate
+// the direct solution up to rounding, so a solve takes one or two
+// iterations.  The scalars stay on the device; the host reads them once per
+// iteration.
 int Domain::solve_wide(int R, const double* const* b, double* const* x, const CgBufs& w, bool graphs,
                        unsigned warm) {
   const int n = num.neq;
   const double tol2 = rtol * rtol;
-  double* vr[2] = {w.r0, wb_v.p};
-  double* vz[2] = {w.z, wb_v.p + n};
-  double* vp[2] = {w.p, wb_v.p + 2 * (size_t)n};
-  double* vq[2] = {w.q, wb_v.p + 3 * (size_t)n};
-  double bb[2] = {0, 0}, rz[2] = {0, 0}, rr[2] = {0, 0};
-  bool conv[2] = {true, true}, fail[2] = {false, false};
-  int its[2] = {0, 0};
+  TilePcg P;
+  P.S = tl_scal.p;
+  P.v[0] = TileRhs{b[0], x[0], w.r0, w.z, w.p, w.q, (int)(warm & 1u)};
+  P.v[1] = R > 1 ? TileRhs{b[1], x[1], tl_v.p, tl_v.p + n, tl_v.p + 2 * (size_t)n, tl_v.p + 3 * (size_t)n,
+                           (int)(warm >> 1 & 1u)}
+                 : P.v[0];
+  auto read = [&] {
+    XG_HIP(hipMemcpyAsync(tl_read, tl_scal.p, R * sizeof(TileScal), hipMemcpyDeviceToHost, stream));
+    XG_HIP(hipStreamSynchronize(stream));
+  };
   for (int s = 0; s < R; s++) {
-    launch_copy(stream, n, b[s], vr[s]);
-    bb[s] = dot_dev(b[s], b[s], n);
-    conv[s] = !(bb[s] > 0);
-    if (!((warm >> s) & 1u) || conv[s]) {
-      wband_zero(stream, n, x[s]);
-    } else {
-      // from the guess in x (bit s of warm): r = b - A x; a guess already
-      // within the tolerance ends the solve before the first iteration
-      spmv(x[s], vq[s], true);
-      launch_axpby(stream, n, -1.0, vq[s], 1.0, vr[s]);
-      rr[s] = dot_dev(vr[s], vr[s], n);
-      conv[s] = rr[s] <= tol2 * bb[s];
-    }
+    tl_read[s].conv = 0;
+    if (P.v[s].warm) spmv(x[s], P.v[s].q, true);
   }
-  auto apply_open = [&] {
+  tiles_pcg_start(stream, n, R, P, tol2);
+  if (warm) read();  // a guess within the tolerance ends its solve before the first iteration
+  for (int it = 0; it < maxit; it++) {
     const double* rs[2];
     double* zs[2];
     int k = 0;
     for (int s = 0; s < R; s++)
-      if (!conv[s]) {
-        rs[k] = vr[s];
-        zs[k] = vz[s];
-        k++;
+      if (!tl_read[s].conv) {
+        rs[k] = P.v[s].r;
+        zs[k++] = P.v[s].z;
       }
-    if (k) wb_apply(k, rs, zs, graphs);
-  };
-  apply_open();
-  for (int s = 0; s < R; s++)
-    if (!conv[s]) {
-      rz[s] = dot_dev(vr[s], vz[s], n);
-      launch_copy(stream, n, vz[s], vp[s]);
-    }
-  for (int it = 0; it < maxit && !(conv[0] && conv[1]); it++) {
-    for (int s = 0; s < R; s++) {
-      if (conv[s]) continue;
-      its[s]++;
-      spmv(vp[s], vq[s], true);
-      const double pq = dot_dev(vp[s], vq[s], n);
-      if (pq == 0.0 || !std::isfinite(pq)) {
-        conv[s] = fail[s] = true;
-        continue;
-      }
-      const double alpha = rz[s] / pq;
-      launch_axpby(stream, n, alpha, vp[s], 1.0, x[s]);
-      launch_axpby(stream, n, -alpha, vq[s], 1.0, vr[s]);
-      rr[s] = dot_dev(vr[s], vr[s], n);
-      if (rr[s] <= tol2 * bb[s]) conv[s] = true;
-    }
-    if (conv[0] && conv[1]) break;
-    apply_open();
-    for (int s = 0; s < R; s++) {
-      if (conv[s]) continue;
-      const double rzn = dot_dev(vr[s], vz[s], n);
-      const double beta = rzn / rz[s];
-      rz[s] = rzn;
-      launch_axpby(stream, n, 1.0, vz[s], beta, vp[s]);
-    }
+    if (k == 0) break;
+    tiles_apply(k, rs, zs, graphs);
+    tiles_pcg_dir(stream, n, R, P);
+    for (int s = 0; s < R; s++)
+      if (!tl_read[s].conv) spmv(P.v[s].p, P.v[s].q, true);
+    tiles_pcg_step(stream, n, R, P, tol2);
+    read();
   }
   int status = 0;
   for (int s = 0; s < R; s++) {
+    const TileScal& S = tl_read[s];
     counters.solves++;
-    counters.cg_iters += its[s];
-    counters.last_cg_relres = bb[s] > 0 ? std::sqrt(rr[s] / bb[s]) : 0.0;
-    if (fail[s] || (bb[s] > 0 && !(rr[s] <= tol2 * bb[s]))) status = XG_BAD_LINEAR_SOLVE;
+    counters.cg_iters += S.iters;
+    counters.last_cg_relres = S.bb > 0 ? std::sqrt(S.rr / S.bb) : 0.0;
+    if (S.fail || (S.bb > 0 && !(S.rr <= tol2 * S.bb))) status = XG_BAD_LINEAR_SOLVE;
   }
   return status;
+}
+
+// Takes the system into the tiled factorisation where its plan fits: builds
+// the plan (xg_tileplan.h) and the device arrays of its launches.
+void Domain::tiles_setup(int bw) {
+  TilePlan P;
+  const int n = num.neq;
+  const long long max_tiles = (long long)(kTileMaxBytes / (sizeof(double) * kTile * kTile));
+  if (!tile_plan(n, num.rowptr, num.colind, nnode, ndf, ndm, num.eq, crd_h, max_tiles, 1e300, P)) return;
+  // panel tasks: a workgroup per row tile, several where a level has many
+  // (every workgroup of a column inverts its diagonal block itself)
+  std::vector<int4> task;
+  TileHost& H = tl_host;
+  H = TileHost{};
+  H.tiles = P.tiles();
+  H.upptr = P.upptr;
+  H.fwptr = P.fwptr;
+  H.bwptr = P.bwptr;
+  H.panptr.assign(1, 0);
+  for (int l = 0; l < P.nlev; l++) {
+    int rows = 0;
+    for (int c = P.levptr[l]; c < P.levptr[l + 1]; c++)
+      rows += P.colptr[P.levcol[c] + 1] - P.colptr[P.levcol[c]];
+    const int chunk = std::max(1, (rows + kTilePanelGroups - 1) / kTilePanelGroups);
+    for (int c = P.levptr[l]; c < P.levptr[l + 1]; c++) {
+      const int k = P.levcol[c], m = P.colptr[k + 1] - P.colptr[k];
+      int j = 0;
+      do {
+        task.push_back(int4{k, j, std::min(chunk, m - j), 0});
+        j += chunk;
+      } while (j < m);
+    }
+    H.panptr.push_back((int)task.size());
+  }
+  std::vector<int> ipos((size_t)kTile * P.nt, -1), all;
+  for (int e = 0; e < n; e++) ipos[P.pos[e]] = e;
+  std::vector<std::pair<const int**, const std::vector<int>*>> parts = {
+      {&tl_view.pos, &P.pos},     {&tl_view.ipos, &ipos},     {&tl_view.wid, &P.wid},     {&tl_view.colptr, &P.colptr},
+      {&tl_view.row, &P.row},     {&tl_view.uptgt, &P.uptgt}, {&tl_view.upsrc, &P.upsrc},
+      {&tl_view.srcg, &P.srcg},   {&tl_view.srca, &P.srca},   {&tl_view.srck, &P.srck},   {&tl_view.fwrow, &P.fwrow},
+      {&tl_view.fwsrc, &P.fwsrc}, {&tl_view.fwg, &P.fwg},     {&tl_view.fwk, &P.fwk},     {&tl_view.bwcol, &P.bwcol},
+      {&tl_view.bwsrc, &P.bwsrc}, {&tl_view.bwg, &P.bwg},     {&tl_view.bwr, &P.bwr}};
+  for (auto& q : parts) all.insert(all.end(), q.second->begin(), q.second->end());
+  tl_ints.upload(all, stream);
+  tl_task.upload(task, stream);
+  XG_HIP(hipStreamSynchronize(stream));
+  size_t off = 0;
+  for (auto& q : parts) {
+    *q.first = tl_ints.p + off;
+    off += q.second->size();
+  }
+  tl_view.task = tl_task.p;
+  tl_view.nt = P.nt;
+  const size_t doubles = (size_t)P.tiles() * kTile * kTile, np = (size_t)kTile * P.nt;
+  tl_A.resize(doubles);
+  tl_G.resize(doubles);
+  tl_Y.resize(2 * np);
+  tl_X.resize(2 * np);
+  tl_v.resize(4 * (size_t)n);
+  tl_scal.resize(2);
+  if (!tl_read) XG_HIP(hipHostMalloc((void**)&tl_read, 2 * sizeof(TileScal), hipHostMallocDefault));
+  tl_bw = bw;
 }
 
 // Half bandwidth of the pattern under an equation order (pinv: position of
@@ -1006,7 +1035,7 @@ static int band_width(const Numbering& num, const std::vector<int>& pinv) {
 
 void Domain::band_order() {
   band_bw = -1;
-  wb_bw = -1;
+  tl_bw = -1;
   pc_cache = pc_fresh = false;
   pc_vals.release();
   pc_diff.release();
@@ -1015,9 +1044,12 @@ void Domain::band_order() {
   band2.release();
   band_L.release();
   band_Lr.release();
-  for (auto* v : {&wb_L, &wb_D, &wb_Y, &wb_v}) v->release();
+  for (auto* v : {&tl_A, &tl_G, &tl_Y, &tl_X, &tl_v}) v->release();
+  tl_ints.release();
+  tl_task.release();
+  tl_view = TileView{};
   const int n = num.neq;
-  if (n == 0 || n > kWbMaxEqn) return;
+  if (n == 0 || n > kTileMaxEqn) return;
   std::vector<int> ident(n);
   for (int i = 0; i < n; i++) ident[i] = i;
   int best = band_width(num, ident);
@@ -1055,22 +1087,9 @@ void Domain::band_order() {
       pinv = geo;
     }
   }
-  if (best > 63 || n > kBandMaxEqn) {
-    // the tiled factor of xg_wband.hip, for systems the one-workgroup
-    // solve does not take
-    if (n <= 1024 || best > kWbMaxBw) return;
-    const size_t np = (size_t)wband_padded(n);
-    const size_t need = (wband_factor_doubles(n, best) + wband_diag_doubles(n) + 6 * np + 4 * (size_t)n) * 8;
-    if (need > kWbMaxBytes) return;
-    wb_bw = best;
-    band_pinv.upload(pinv, stream);
-    wb_L.resize(wband_factor_doubles(n, best));
-    wb_D.resize(wband_diag_doubles(n));
-    wb_Y.resize(6 * np);
-    wb_v.resize(4 * (size_t)n);
-    pc_buffers();
-    return;
-  }
+  if (n >= kTileMinEqn) tiles_setup(best);
+  if (tl_bw >= 0) pc_buffers();
+  if (best > 63 || n > kBandMaxEqn) return;
   band_bw = best;
   band_pinv.upload(pinv, stream);
   band_A.resize((size_t)n * (best + 1));
@@ -1097,8 +1116,8 @@ void Domain::pc_buffers() {
 void Domain::cg_graph_clear() {
   for (auto& g : cg_graphs) destroy_graph(stream, g.graph, g.exec);
   cg_graphs.clear();
-  destroy_graph(stream, wb_fg, wb_fe);
-  for (int k = 0; k < 2; k++) destroy_graph(stream, wb_sg[k], wb_se[k]);
+  destroy_graph(stream, tl_fg, tl_fe);
+  for (int k = 0; k < 2; k++) destroy_graph(stream, tl_sg[k], tl_se[k]);
 }
 
 // One chunk of PCG iterations.  A chunk of an even length starting on an
@@ -1153,7 +1172,7 @@ void Domain::cg_chunk_run(int iters, int it0, int L, int bw, double* x, const Cg
 // results); otherwise one after the other.
 int Domain::solve_pair(const double* b1, double* x1, const double* b2, double* x2) {
   const int n = num.neq;
-  if (n > 0 && !small_path() && wide_active()) {
+  if (n > 0 && wide_active()) {
     const CgBufs w = cg_bufs();
     if (!precond_ready(w)) return XG_BAD_LINEAR_SOLVE;
     if (wide_active()) {
@@ -1202,7 +1221,7 @@ int Domain::solve_pair(const double* b1, double* x1, const double* b2, double* x
 // that met a pivot that is not positive gives way to the PCG without it.
 bool Domain::precond_ready(const CgBufs& w) {
   for (;;) {
-    const bool wide = band_active() || (w.wide && wide_active() && !small_path());
+    const bool exact = band_active() || wide_active();
     precond_setup(w);
     int bad = 0;
     XG_HIP(hipMemcpyAsync(&bad, w.pcbad, sizeof(int), hipMemcpyDeviceToHost, stream));
@@ -1217,7 +1236,7 @@ bool Domain::precond_ready(const CgBufs& w) {
       return true;
     }
     pc_fresh = false;
-    if (!wide) return false;
+    if (!exact) return false;
     wb_failed = true;
     wb_fallbacks++;
     pc_done = nullptr;
@@ -1237,7 +1256,7 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
     cg_solve_band(stream, n, rowptr.p, colind.p, vals.p, band_bw, band_pinv.p, w.bandL, w.bandLr, rtol * rtol, maxit,
                   R);
     cg_read_scal(stream, w.scal, &conv, &it, &rr, &bb, &brk);
-  } else if (!small_path() && w.wide && wide_active()) {
+  } else if (wide_active()) {
     const double* bs[1] = {b};
     double* xs[1] = {x};
     return solve_wide(1, bs, xs, w, graphs, warm ? 1u : 0u);
@@ -1457,7 +1476,7 @@ int Domain::newton() {
   bool first = true;
   do {
     form_tangent();
-    if (integ == 2 && (band_active() || (wide_active() && !small_path()))) {
+    if (integ == 2 && (band_active() || wide_active())) {
       // DisplacementControl::update solves for the reference load with the
       // same matrix: both solves at once
       if (solve_pair(B.p, X.p, phat.p, dUhat.p) < 0) return XG_BAD_LINEAR_SOLVE;

@@ -11,6 +11,7 @@
 #include "xg_kernels.h"
 #include "xg_memory.h"
 #include "xg_numbering.h"
+#include "xg_tiles.h"
 
 namespace xg {
 
@@ -215,7 +216,6 @@ struct Domain {
     void* scal;
     double *bandA, *bandL, *bandLr;  // band matrix and its Cholesky factor (band_active())
     double *bs = nullptr, *xs = nullptr, *binvs = nullptr;  // b, x and binv in the sweep order (sym_sweep)
-    bool wide = false;  // the domain's wide-band factor may be used (wide_active())
   };
   // the symmetric product in its sweep order runs this solve (chunked PCG)
   bool sweep_active(const CgBufs& w) { return sym_sweep && w.bs && w.xs && w.binvs && sym_prepare(true); }
@@ -232,24 +232,28 @@ struct Domain {
   DVec<char> scal2;
   bool dc_hat_ready = false;  // the Newton iteration has solved for the reference load
   int solve_pair(const double* b1, double* x1, const double* b2, double* x2);
-  bool band_active() const { return cg_small_on && band_bw >= 0 && !wb_failed; }
+  bool band_active() const { return cg_small_on && band_bw >= 0 && !wb_failed && !wide_active(); }
   void band_order();
-  // band-Cholesky preconditioner of wider bands (xg_wband.hip): systems of
-  // more than 1,024 equations (the one-workgroup solve takes smaller ones)
-  // whose half bandwidth in the band order is at most kWbMaxBw, or at most
-  // 63 with more than kBandMaxEqn equations, and whose factor fits in
-  // kWbMaxBytes, under the static integrators (a transient's K + c3 M is
-  // well conditioned by the mass term: block Jacobi converges in tens of
-  // iterations there, faster than a factorisation per Newton iteration).
-  // The PCG preconditioned by the exact factor converges in one or two
+  // tiled sparse factorisation (xg_tiles.hip), the exact preconditioner
+  // under the static integrators of the systems tiles_setup() takes (a
+  // transient's K + c3 M is well conditioned by the mass term: block Jacobi
+  // converges in tens of iterations there).  A solve takes one or two PCG
   // iterations (solve_wide); factor and sweeps are replayed from captured
   // graphs when cg_graph_on.
-  static constexpr int kWbMaxEqn = 1 << 18;
-  static constexpr size_t kWbMaxBytes = size_t(1) << 30;
-  int wb_bw = -1;
-  DVec<double> wb_L, wb_D, wb_Y, wb_v;  // factor tiles, diagonal tiles, 3 x 2 sweep vectors, 4 PCG vectors
-  hipGraph_t wb_fg = nullptr, wb_sg[2] = {nullptr, nullptr};
-  hipGraphExec_t wb_fe = nullptr, wb_se[2] = {nullptr, nullptr};
+  static constexpr int kTileMinEqn = 385, kTileMaxEqn = 1 << 18;
+  static constexpr int kTilePanelGroups = 512;
+  static constexpr size_t kTileMaxBytes = size_t(1) << 30;  // each of A and G
+  int tl_bw = -1;  // half bandwidth in the band order (reported), -1: no plan
+  TileView tl_view;
+  TileHost tl_host;
+  DVec<int> tl_ints;
+  DVec<int4> tl_task;
+  DVec<double> tl_A, tl_G, tl_Y, tl_X, tl_v;  // tiles, sweep vectors, 4 PCG vectors of a second right-hand side
+  DVec<TileScal> tl_scal;
+  TileScal* tl_read = nullptr;  // pinned copy of tl_scal
+  hipGraph_t tl_fg = nullptr, tl_sg[2] = {nullptr, nullptr};
+  hipGraphExec_t tl_fe = nullptr, tl_se[2] = {nullptr, nullptr};
+  void tiles_setup(int bw);
   bool cg_wide_on = true;
   // the current matrix's band factor (either kind) met a pivot that is not
   // positive (an indefinite tangent past a peak): its solves fall back to
@@ -266,12 +270,10 @@ struct Domain {
   const void* pc_cache_key = nullptr;
   const void* pc_fresh_key = nullptr;
   long long pc_reuses = 0;
-  bool wide_active() const {
-    return cg_small_on && cg_wide_on && !wb_failed && wb_bw >= 0 && band_bw < 0 && integ != 3;
-  }
-  void wb_factor(int* bad);
+  bool wide_active() const { return cg_small_on && cg_wide_on && !wb_failed && tl_bw >= 0 && integ != 3; }
+  void tiles_form(int* bad);
   void pc_buffers();
-  void wb_apply(int k, const double* const* r, double* const* z, bool graphs);
+  void tiles_apply(int k, const double* const* r, double* const* z, bool graphs);
   // warm: bit s set when x[s] holds a guess to start right-hand side s from
   int solve_wide(int R, const double* const* b, double* const* x, const CgBufs& w, bool graphs, unsigned warm = 0);
   // the preconditioner's buffers last formed from the current matrix
@@ -318,7 +320,9 @@ struct Domain {
   // sym_sweep, else the equation order)
   void spmv_sweep(const double* x, double* y);
   // the whole solve runs in one workgroup (k_pcg_small)
-  bool small_path() const { return cg_small_on && cg_small_fits(num.neq, (long long)num.colind.size()); }
+  bool small_path() const {
+    return cg_small_on && !wide_active() && cg_small_fits(num.neq, (long long)num.colind.size());
+  }
 };
 
 // no-allocation solve (xg_noalloc.cpp): per-device scratch lookup at

@@ -279,9 +279,9 @@ class Model:
         iteration, sums in another order), and whether the first Newton
         iteration of a step (and DisplacementControl's reference-load solve)
         starts from the previous step's solution instead of zero (the same
-        tolerance, fewer iterations), and whether systems of more than 1,024
-        equations with a band of at most 1,024 are preconditioned by their
-        exact tiled band factor (with small)."""
+        tolerance, fewer iterations), and whether systems of 385 equations
+        and more are preconditioned by their exact tiled sparse factor under
+        the static integrators, where it fits (with small)."""
         flags = (int(bool(graph)) | 2 * int(bool(fuse)) | 4 * int(bool(small)) | 8 * int(bool(warm))
                  | 16 * int(bool(wide)))
         self._check(self._b.cg_config(self._h, int(chunk), flags))
