@@ -72,7 +72,9 @@ def check_indices(P, n):
             s = slice(P["upsrc"][i], P["upsrc"][i + 1])
             g, a, tgt = P["srcg"][s], P["srca"][s], P["uptgt"][i]
             assert len(g) and g.max() < slots and tgt < slots
-            assert np.all(P["lev"][col_of[g]] == l) and np.array_equal(col_of[g], col_of[a])
+            # from this level's columns, or earlier ones of a run that ends in it
+            assert np.all(P["lev"][col_of[g]] <= l) and np.array_equal(col_of[g], col_of[a])
+            assert P["lev"][col_of[tgt]] > l and np.all(np.diff(col_of[g]) > 0)
             assert np.all(row_of[g] == row_of[tgt]) and np.all(row_of[a] == col_of[tgt])
             assert np.all(g != a + 0 * g) or row_of[tgt] == col_of[tgt]
             assert np.array_equal(P["srck"][s], (P["wid"][col_of[g]] + 15) // 16 * 16)

@@ -5,9 +5,12 @@
 #include "xg_domain.h"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <future>
+#include <system_error>
 
 #include "xg_frame.h"
 #include "xg_j2.h"
@@ -213,7 +216,13 @@ struct J2Group : Group {
 // ---------------------------------------------------------------------------
 // Domain
 // ---------------------------------------------------------------------------
+struct Domain::TilePlanJob {
+  TilePlan plan;
+  std::future<bool> done;
+};
+
 Domain::~Domain() {
+  if (tl_job && tl_job->done.valid()) tl_job->done.wait();
   cg_graph_clear();
   if (tl_read) (void)hipHostFree(tl_read);
   if (ev0) (void)hipEventDestroy(ev0);
@@ -527,6 +536,7 @@ void Domain::setup() {
   number_and_pattern(nnode, ndf, fixed, elem_nodes, numberer == XG_NUMBERER_RCM, num);
   const int neq = num.neq;
   const long long nnz = (long long)num.colind.size();
+  tiles_plan_start();
   // element matrix / vector offsets
   ke_total = re_total = 0;
   for (auto& g : groups) {
@@ -961,13 +971,40 @@ int Domain::solve_wide(int R, const double* const* b, double* const* x, const Cg
   return status;
 }
 
-// Takes the system into the tiled factorisation where its plan fits: builds
-// the plan (xg_tileplan.h) and the device arrays of its launches.
-void Domain::tiles_setup(int bw) {
-  TilePlan P;
+// Starts the tiled factorisation's plan (host code) on a thread of its own:
+// it reads the numbering and the coordinates, which the rest of the set-up
+// leaves alone.  Without a thread to spare it runs here.
+void Domain::tiles_plan_start() {
+  if (tl_job && tl_job->done.valid()) tl_job->done.wait();  // of a set-up that threw
+  tl_job.reset();
   const int n = num.neq;
-  const long long max_tiles = (long long)(kTileMaxBytes / (sizeof(double) * kTile * kTile));
-  if (!tile_plan(n, num.rowptr, num.colind, nnode, ndf, ndm, num.eq, crd_h, max_tiles, 1e300, P)) return;
+  if (n < kTileMinEqn || n > kTileMaxEqn) return;
+  tl_job = std::make_shared<TilePlanJob>();
+  TilePlanJob* job = tl_job.get();
+  auto build = [this, n, job] {
+    const long long max_tiles = (long long)(kTileMaxBytes / (sizeof(double) * kTile * kTile));
+    return tile_plan(n, num.rowptr, num.colind, nnode, ndf, ndm, num.eq, crd_h, max_tiles, 1e300, job->plan);
+  };
+  try {
+    job->done = std::async(std::launch::async, build);
+  } catch (const std::system_error&) {
+    job->done = std::async(std::launch::deferred, build);
+  }
+}
+
+// Takes the system into the tiled factorisation where its plan fits: the
+// device arrays of its launches.
+void Domain::tiles_setup(int bw) {
+  if (!tl_job) return;
+  const bool ok = tl_job->done.get();
+  const TilePlan P = std::move(tl_job->plan);
+  tl_job.reset();
+  if (!ok) return;
+  const int n = num.neq;
+  tl_factor_us = 25.0 * P.nlev + P.flops / 30e6;
+  tl_iter_us = 15.0 + 0.55 * 8.0 * (double)num.colind.size() / 3.4e6;
+  tl_cap = std::max(cg_chunk, (int)(tl_factor_us / tl_iter_us));
+  tl_on = false;
   // panel tasks: a workgroup per row tile, several where a level has many
   // (every workgroup of a column inverts its diagonal block itself)
   std::vector<int4> task;
@@ -1036,6 +1073,7 @@ static int band_width(const Numbering& num, const std::vector<int>& pinv) {
 void Domain::band_order() {
   band_bw = -1;
   tl_bw = -1;
+  tl_factor_us = 0;
   pc_cache = pc_fresh = false;
   pc_vals.release();
   pc_diff.release();
@@ -1087,7 +1125,7 @@ void Domain::band_order() {
       pinv = geo;
     }
   }
-  if (n >= kTileMinEqn) tiles_setup(best);
+  tiles_setup(best);
   if (tl_bw >= 0) pc_buffers();
   if (best > 63 || n > kBandMaxEqn) return;
   band_bw = best;
@@ -1282,6 +1320,7 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
     cg_start(stream, n, bs, xs, w.r0, w.z, w.p, bw, sweep ? w.binvs : w.binv, bfirst.p, bsize.p, w.part,
              rtol * rtol, maxit, w.scal, warm ? w.q : nullptr);
     int issued = 0, next = cg_chunk;
+    const int cap = tl_usable() && tl_big() && !tl_on ? tl_cap : INT_MAX;
     const int L = lanes();
     while (true) {
       cg_read_scal(stream, w.scal, &conv, &it, &rr, &bb, &brk);
@@ -1291,6 +1330,12 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
       // iteration later (the extra iteration then returns at once, as it
       // does on the other path, where the test ends the iteration)
       if (issued >= maxit + 1) break;
+      if (issued >= cap) {
+        // worth a factor: this solve again, and the later ones, with it
+        counters.cg_iters += it;
+        tl_on = true;
+        return solve_with(b, x, w, graphs);
+      }
       // chunks double (up to 8x cg_chunk) while the solve goes on: fewer
       // host round trips on long solves; iterations issued past
       // convergence return at once
@@ -1348,6 +1393,7 @@ void Domain::revert_to_start() {
   A.zero(stream);
   Ac.zero(stream);
   for (auto& g : groups) g->revert_to_start(*this);
+  tl_on = false;
   lambda = 0;
   time = 0;
   const double dt_keep = dt;

@@ -242,7 +242,26 @@ struct Domain {
   // graphs when cg_graph_on.
   static constexpr int kTileMinEqn = 385, kTileMaxEqn = 1 << 18;
   static constexpr int kTilePanelGroups = 512;
-  static constexpr size_t kTileMaxBytes = size_t(1) << 30;  // each of A and G
+  static constexpr size_t kTileMaxBytes = size_t(4) << 30;  // each of A and G
+  // A large solid's factor takes as long as hundreds of PCG iterations
+  // (tl_factor_us, tl_iter_us: fits to solids of 12^3 to 33^3 elements, 25 us
+  // per level and 30 TFLOP/s; 15 us per iteration and 3.4 TB/s of the
+  // product).  Above kTileBigUs such a model starts with block Jacobi, and a
+  // solve that has not converged after as many iterations as a factor is
+  // worth (tl_cap) goes on with the factor, as do the later ones until
+  // revertToStart: at most twice the better of the two on any solve, and
+  // mildly plastic steps (100 to 300 iterations at 28 us on 33^3) keep the
+  // cheap iterations where the factor takes 16 ms.
+  static constexpr double kTileBigUs = 3000.0;
+  double tl_factor_us = 0, tl_iter_us = 1;
+  bool tl_on = false;  // a solve has gone on with the factor
+  int tl_cap = 0;
+  bool tl_big() const { return tl_factor_us > kTileBigUs; }
+  bool tl_usable() const { return cg_small_on && cg_wide_on && !wb_failed && tl_bw >= 0 && integ != 3; }
+  // the plan, built beside the rest of the set-up
+  struct TilePlanJob;
+  std::shared_ptr<TilePlanJob> tl_job;
+  void tiles_plan_start();
   int tl_bw = -1;  // half bandwidth in the band order (reported), -1: no plan
   TileView tl_view;
   TileHost tl_host;
@@ -270,7 +289,7 @@ struct Domain {
   const void* pc_cache_key = nullptr;
   const void* pc_fresh_key = nullptr;
   long long pc_reuses = 0;
-  bool wide_active() const { return cg_small_on && cg_wide_on && !wb_failed && tl_bw >= 0 && integ != 3; }
+  bool wide_active() const { return tl_usable() && (!tl_big() || tl_on); }
   void tiles_form(int* bad);
   void pc_buffers();
   void tiles_apply(int k, const double* const* r, double* const* z, bool graphs);

@@ -20,6 +20,13 @@
 //
 // Levels.  level(k) = 1 + the highest level of a column whose factor updates
 // column k; the columns of one level are independent.
+//
+// Groups.  Runs of up to kTileGroup columns of one piece in which each
+// updates the next: inside a run a column's update is applied at its level,
+// to the tiles beyond the run all its columns' at the level of the last one,
+// in one pass over each target.  (Every tile that a column of the run updates
+// beyond it lies in a column of a higher level than the run's last, which
+// has inherited the run's rows.)
 #pragma once
 #include <algorithm>
 #include <cstdint>
@@ -28,6 +35,7 @@
 namespace xg {
 
 constexpr int kTile = 64;
+constexpr int kTileGroup = 4;
 
 struct TilePlan {
   int nt = 0;                 // tile columns
@@ -270,6 +278,7 @@ inline bool tile_plan(int n, const std::vector<int>& rowptr, const std::vector<i
   P.pos.assign(n, -1);
   std::vector<int> col_of(n);
   size_t b = 0;
+  std::vector<int> piece;  // of each tile column
   for (int en : ends) {
     int fill = kTile;
     for (; b < (size_t)en; b++)
@@ -278,6 +287,7 @@ inline bool tile_plan(int n, const std::vector<int>& rowptr, const std::vector<i
         if (e < 0) continue;
         if (fill == kTile) {
           P.wid.push_back(0);
+          piece.push_back(en);
           fill = 0;
         }
         col_of[e] = (int)P.wid.size() - 1;
@@ -351,23 +361,35 @@ inline bool tile_plan(int n, const std::vector<int>& rowptr, const std::vector<i
   struct Src {
     int tgt, g, a, k;
   };
-  std::vector<Src> up, fw;
+  // last column of each column's group
+  std::vector<int> last(nt);
+  for (int k = nt - 1, left = 0; k >= 0; k--) {
+    const bool chain = k + 1 < nt && piece[k + 1] == piece[k] && !str[k].empty() && str[k][0] == k + 1;
+    left = chain && left > 1 ? left - 1 : kTileGroup;
+    last[k] = left < kTileGroup ? last[k + 1] : k;
+  }
+  std::vector<Src> fw;
+  std::vector<std::vector<Src>> ups(P.nlev);
+  for (int k = 0; k < nt; k++) {
+    const std::vector<int>& s = str[k];
+    const int base = (int)P.diag(k) + 1;
+    for (size_t b2 = 0; b2 < s.size(); b2++)
+      for (size_t a2 = b2; a2 < s.size(); a2++)
+        ups[P.lev[s[b2] <= last[k] ? k : last[k]]].push_back(
+            {slot(s[a2], s[b2]), base + (int)a2, base + (int)b2, k});
+  }
   P.upptr.assign(1, 0);
   P.fwptr.assign(1, 0);
   P.upsrc.assign(1, 0);
   P.fwsrc.assign(1, 0);
   for (int l = 0; l < P.nlev; l++) {
-    up.clear();
+    std::vector<Src>& up = ups[l];
     fw.clear();
     for (int c = P.levptr[l]; c < P.levptr[l + 1]; c++) {
       const int k = P.levcol[c];
       const std::vector<int>& s = str[k];
       const int base = (int)P.diag(k) + 1;
-      for (size_t b2 = 0; b2 < s.size(); b2++) {
-        fw.push_back({s[b2], base + (int)b2, 0, k});
-        for (size_t a2 = b2; a2 < s.size(); a2++)
-          up.push_back({slot(s[a2], s[b2]), base + (int)a2, base + (int)b2, k});
-      }
+      for (size_t b2 = 0; b2 < s.size(); b2++) fw.push_back({s[b2], base + (int)b2, 0, k});
     }
     auto less = [](const Src& x, const Src& y) { return x.tgt != y.tgt ? x.tgt < y.tgt : x.k < y.k; };
     std::sort(up.begin(), up.end(), less);
