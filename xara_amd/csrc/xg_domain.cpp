@@ -1300,8 +1300,8 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
     return solve_wide(1, bs, xs, w, graphs, warm ? 1u : 0u);
   } else if (small_path()) {
     // the whole solve in one workgroup, one launch
-    cg_solve_small(stream, n, rowptr.p, colind.p, vals.p, b, x, w.r0, w.z, w.p, w.q, bw, w.binv, bfirst.p, bsize.p,
-                   rtol * rtol, maxit, w.scal);
+    cg_solve_small(stream, n, (long long)num.colind.size(), rowptr.p, colind.p, vals.p, b, x, bw, w.binv, bfirst.p,
+                   bsize.p, rtol * rtol, maxit, w.scal);
     cg_read_scal(stream, w.scal, &conv, &it, &rr, &bb, &brk);
   } else {
     // in the sweep order of the symmetric product: b (and a warm start's

@@ -130,9 +130,9 @@ void cg_solve_band(hipStream_t s, int n, const int* rowptr, const int* colind, c
                    const BandRhs* r1 = nullptr);
 // whole solve in one workgroup (k_pcg_small) for systems that fit it
 bool cg_small_fits(int n, long long nnz);
-void cg_solve_small(hipStream_t s, int n, const int* rowptr, const int* colind, const double* vals, const double* b,
-                    double* x, double* r, double* z, double* p, double* q, int bw, const double* binv,
-                    const int* bfirst, const unsigned char* bsize, double tol2, int maxit, void* scal);
+void cg_solve_small(hipStream_t s, int n, long long nnz, const int* rowptr, const int* colind, const double* vals,
+                    const double* b, double* x, int bw, const double* binv, const int* bfirst,
+                    const unsigned char* bsize, double tol2, int maxit, void* scal);
 void cg_read_scal(hipStream_t s, const void* scal, int* converged, int* iter, double* rr, double* bb,
                   int* breakdown);
 

@@ -736,14 +736,41 @@ __global__ __launch_bounds__(256) void k_cg_init_scal(int nb, const double* __re
 // alpha = r.z / p.q, beta = r.z (new) / r.z (old), stop when r.r <= tol2 b.b
 // or after maxit iterations, breakdown on a zero or non-finite p.q), with
 // workgroup barriers in place of kernel boundaries and no host round trip
-// per chunk: a few microseconds per iteration where five (or three) launches
-// per iteration take tens.  Thread t owns rows t, t + 1024, ...; sums go
-// through a fixed wave butterfly and a fixed pass over the 16 wave sums, so
-// every thread holds the same bits and takes the same branches.  The final
-// scalars go to the CGScal the host reads.
+// per chunk.  G lanes to a row (G n <= 1,024): each keeps its first K entries
+// in registers for the whole solve, with their columns, reads further ones
+// from memory, and takes p from LDS; K is what the registers of NT threads
+// hold (44 for 768 threads, 24 for 1,024). the row's first lane owns
+// its x, r, p and row of the block inverse.  Sums go through a fixed order
+// of lanes and wavefronts, so every thread holds the same bits and takes the
+// same branches.  The final scalars go to the CGScal the host reads.
+//
+// Bound by the four barriers of an iteration and the LDS reads between them.
+// With a thread per row and matrix and vectors in memory, the pushover of a
+// 4^3 solid (300 equations, 765 iterations) took 14.9 ms, now 4.3; that of a
+// 288-equation frame (2,471 iterations) 32.4 ms, now 12.3.
 // ---------------------------------------------------------------------------
 constexpr int kSmallPcgThreads = 1024;
 
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_at(double v, int l) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
+  return __hiloint2double(hi, lo);
+}
+// the wavefront's total: pairs, quads, half rows and rows by DPP, then the
+// four rows in order
+__device__ __forceinline__ double wave_total(double v) {
+  v += dpp_d<0xB1>(v);   // lane ^ 1
+  v += dpp_d<0x4E>(v);   // lane ^ 2
+  v += dpp_d<0x141>(v);  // mirror of the half row
+  v += dpp_d<0x140>(v);  // mirror of the row
+  return ((wave_at(v, 0) + wave_at(v, 16)) + wave_at(v, 32)) + wave_at(v, 48);
+}
 __device__ __forceinline__ double block_sum_1024(double v, double* sh) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -756,102 +783,126 @@ __device__ __forceinline__ double block_sum_1024(double v, double* sh) {
   return s;
 }
 
-template <int BW>
-__device__ __forceinline__ double small_precond(int i, const double* __restrict__ r, const double* __restrict__ binv,
-                                                const int* __restrict__ bfirst,
-                                                const unsigned char* __restrict__ bsize) {
-  if constexpr (BW == 1) {
-    return binv[i] * r[i];
-  } else {
-    const int f = bfirst[i], m = bsize[i];
-    double zi = 0.0;
+// totals over the workgroup's nw wavefronts of two values, one barrier; sh
+// (2 x 16) must not be written again before the next barrier
+__device__ __forceinline__ void small_sums(double& a, double& b, int nw, double* sh) {
+  a = wave_total(a);
+  b = wave_total(b);
+  if ((threadIdx.x & 63) == 0) {
+    sh[2 * (threadIdx.x >> 6)] = a;
+    sh[2 * (threadIdx.x >> 6) + 1] = b;
+  }
+  __syncthreads();
+  a = 0.0;
+  b = 0.0;
 #pragma unroll
-    for (int j = 0; j < BW; j++)
-      if (j < m) zi += binv[(long long)i * BW + j] * r[f + j];
-    return zi;
+  for (int w = 0; w < kSmallPcgThreads / 64; w++) {
+    const double2 v = *reinterpret_cast<const double2*>(sh + 2 * w);
+    a += w < nw ? v.x : 0.0;
+    b += w < nw ? v.y : 0.0;
   }
 }
 
-template <int BW>
-__global__ __launch_bounds__(kSmallPcgThreads) void k_pcg_small(
-    int n, const int* __restrict__ rowptr, const int* __restrict__ colind, const double* __restrict__ vals,
-    const double* __restrict__ b, double* __restrict__ x, double* __restrict__ r, double* __restrict__ z,
-    double* __restrict__ p, double* __restrict__ q, const double* __restrict__ binv, const int* __restrict__ bfirst,
-    const unsigned char* __restrict__ bsize, double tol2, int maxit, CGScal* __restrict__ S) {
-  __shared__ double sh[kSmallPcgThreads / 64];
-  const int t = threadIdx.x;
-  constexpr int NT = kSmallPcgThreads;
-  for (int i = t; i < n; i += NT) {
-    x[i] = 0.0;
-    r[i] = b[i];
+template <int BW, int NT, int K>
+__global__ __launch_bounds__(NT) void k_pcg_small(
+    int n, int lg, const int* __restrict__ rowptr, const int* __restrict__ colind, const double* __restrict__ vals,
+    const double* __restrict__ b, double* __restrict__ x, const double* __restrict__ binv,
+    const int* __restrict__ bfirst, const unsigned char* __restrict__ bsize, double tol2, int maxit,
+    CGScal* __restrict__ S) {
+  __shared__ __align__(16) double shp[NT];
+  __shared__ __align__(16) double shr[NT + 8];
+  __shared__ __align__(16) double sh[2][2 * kSmallPcgThreads / 64];
+  const int t = threadIdx.x, G = 1 << lg, nw = blockDim.x >> 6;
+  const int row = t >> lg, g = t & (G - 1), i = row < n ? row : n - 1;
+  const bool own = row < n && g == 0;
+  // the row's entries g, g + G, ...: the first K in registers
+  const int kb = rowptr[i] + g, ke = row < n ? rowptr[i + 1] : kb;
+  double av[K];
+  unsigned ac[K / 2];
+#pragma unroll
+  for (int u = 0; u < K; u += 2) {
+    const int k0 = kb + (u << lg), k1 = kb + ((u + 1) << lg);
+    const unsigned c0 = k0 < ke ? (unsigned)colind[k0] : 0u, c1 = k1 < ke ? (unsigned)colind[k1] : 0u;
+    av[u] = k0 < ke ? vals[k0] : 0.0;
+    av[u + 1] = k1 < ke ? vals[k1] : 0.0;
+    ac[u / 2] = c0 | c1 << 16;
   }
+  const int krest = kb + (K << lg);
+  // entries of the wavefront's longest row, for its lanes together
+  int most = ke > kb ? (ke - kb + G - 1) >> lg : 0;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, 64));
+  most = __builtin_amdgcn_readfirstlane(most);
+  double bi[BW];
+  int f = 0;
+  if constexpr (BW == 1) {
+    bi[0] = own ? binv[i] : 0.0;
+    f = i;
+  } else {
+    f = bfirst[i];
+    const int m = bsize[i];
+#pragma unroll
+    for (int j = 0; j < BW; j++) bi[j] = own && j < m ? binv[(long long)i * BW + j] : 0.0;
+  }
+  auto precond = [&] {
+    double z = 0.0;
+#pragma unroll
+    for (int j = 0; j < BW; j++) z += bi[j] * shr[f + j];
+    return z;
+  };
+  double xi = 0.0, ri = own ? b[i] : 0.0;
+  if (t < 8) shr[n + t] = 0.0;  // a short last block reads past n (times 0)
+  if (own) shr[i] = ri;
   __syncthreads();
-  double l1 = 0.0, l2 = 0.0;
-  for (int i = t; i < n; i += NT) {
-    const double zi = small_precond<BW>(i, r, binv, bfirst, bsize);
-    z[i] = zi;
-    p[i] = zi;
-    l1 += r[i] * zi;
-    l2 += r[i] * r[i];
-  }
-  double rz = block_sum_1024(l1, sh);
-  const double bb = block_sum_1024(l2, sh);
+  double zi = precond(), pi = zi;
+  double rz = own ? ri * zi : 0.0, bb = ri * ri;
+  if (own) shp[i] = pi;
+  small_sums(rz, bb, nw, sh[0]);
   double rr = bb, pq = 0.0, alpha = 0.0, beta = 0.0;
   int it = 0, brk = 0;
   bool done = bb == 0.0;
   while (!done) {
-    double lpq = 0.0;
-    for (int i = t; i < n; i += NT) {
-      // sixteen entries' loads in flight at a time, summed in order
-      const int rb = rowptr[i], re = rowptr[i + 1];
-      double s = 0.0;
-      for (int k0 = rb; k0 < re; k0 += 16) {
-        int c[16];
-        double v[16];
+    double s0 = 0.0, s1 = 0.0;
+    double tail = 0.0;
+    for (int k = krest; k < ke; k += G) tail += vals[k] * shp[colind[k]];
 #pragma unroll
-        for (int u = 0; u < 16; u++) {
-          const int k = min(k0 + u, re - 1);
-          c[u] = colind[k];
-          v[u] = vals[k];
-        }
-        double pc[16];
-#pragma unroll
-        for (int u = 0; u < 16; u++) pc[u] = p[c[u]];
-#pragma unroll
-        for (int u = 0; u < 16; u++)
-          if (k0 + u < re) s += v[u] * pc[u];
+    for (int u = 0; u < K; u += 4) {
+      if (u < most) {
+        const double p0 = shp[ac[u / 2] & 0xffffu], p1 = shp[ac[u / 2] >> 16];
+        const double p2 = shp[ac[u / 2 + 1] & 0xffffu], p3 = shp[ac[u / 2 + 1] >> 16];
+        s0 = fma(av[u], p0, s0);
+        s1 = fma(av[u + 1], p1, s1);
+        s0 = fma(av[u + 2], p2, s0);
+        s1 = fma(av[u + 3], p3, s1);
       }
-      q[i] = s;
-      lpq += p[i] * s;
     }
-    pq = block_sum_1024(lpq, sh);
+    double q = (s0 + s1) + tail;
+    for (int o = 1; o < G; o <<= 1) q += __shfl_xor(q, o, 64);
+    pq = own ? pi * q : 0.0;
+    double unused = 0.0;
+    small_sums(pq, unused, nw, sh[1]);
     if (pq == 0.0 || !isfinite(pq)) {
       brk = 1;
       break;
     }
     alpha = rz / pq;
-    for (int i = t; i < n; i += NT) {
-      x[i] += alpha * p[i];
-      r[i] -= alpha * q[i];
-    }
+    xi += alpha * pi;
+    ri -= alpha * q;
+    if (own) shr[i] = ri;
     __syncthreads();
-    l1 = 0.0;
-    l2 = 0.0;
-    for (int i = t; i < n; i += NT) {
-      const double zi = small_precond<BW>(i, r, binv, bfirst, bsize);
-      z[i] = zi;
-      l1 += r[i] * zi;
-      l2 += r[i] * r[i];
-    }
-    const double rzn = block_sum_1024(l1, sh);
-    rr = block_sum_1024(l2, sh);
+    zi = precond();
+    double rzn = own ? ri * zi : 0.0;
+    rr = own ? ri * ri : 0.0;
+    small_sums(rzn, rr, nw, sh[0]);
     it++;
     beta = rzn / rz;
     rz = rzn;
     if (rr <= tol2 * bb || it >= maxit) break;
-    for (int i = t; i < n; i += NT) p[i] = z[i] + beta * p[i];
+    pi = zi + beta * pi;
+    if (own) shp[i] = pi;
     __syncthreads();
   }
+  if (own) x[i] = xi;
   if (t == 0) {
     S->rzp[0] = S->rzp[1] = rz;
     S->pq = pq;
@@ -1844,16 +1895,24 @@ void cg_solve_band(hipStream_t s, int n, const int* rowptr, const int* colind, c
 
 bool cg_small_fits(int n, long long nnz) { return n > 0 && n <= 1024 && nnz <= 32768; }
 
-void cg_solve_small(hipStream_t s, int n, const int* rowptr, const int* colind, const double* vals, const double* b,
-                    double* x, double* r, double* z, double* p, double* q, int bw, const double* binv,
-                    const int* bfirst, const unsigned char* bsize, double tol2, int maxit, void* scal) {
+void cg_solve_small(hipStream_t s, int n, long long nnz, const int* rowptr, const int* colind, const double* vals,
+                    const double* b, double* x, int bw, const double* binv, const int* bfirst,
+                    const unsigned char* bsize, double tol2, int maxit, void* scal) {
   CGScal* S = (CGScal*)scal;
-  const dim3 g(1), blk(kSmallPcgThreads);
+  // lanes per row: twelve entries each, as far as 1,024 threads reach
+  int lg = 0;
+  while ((n << (lg + 1)) <= kSmallPcgThreads && nnz > 12LL * n << lg) lg++;
+  const int nt = ((n << lg) + 63) / 64 * 64;
+  const dim3 g(1), blk(nt);
   switch (bw) {
-#define XG_PS(W)                                                                                              \
-  case W:                                                                                                    \
-    hipLaunchKernelGGL(k_pcg_small<W>, g, blk, 0, s, n, rowptr, colind, vals, b, x, r, z, p, q, binv, bfirst, \
-                       bsize, tol2, maxit, S);                                                               \
+#define XG_PS(W)                                                                                                   \
+  case W:                                                                                                          \
+    if (nt <= 768)                                                                                                 \
+      hipLaunchKernelGGL((k_pcg_small<W, 768, 44>), g, blk, 0, s, n, lg, rowptr, colind, vals, b, x, binv, bfirst,  \
+                         bsize, tol2, maxit, S);                                                                   \
+    else                                                                                                           \
+      hipLaunchKernelGGL((k_pcg_small<W, 1024, 24>), g, blk, 0, s, n, lg, rowptr, colind, vals, b, x, binv, bfirst, \
+                         bsize, tol2, maxit, S);                                                                   \
     break;
     XG_PS(1) XG_PS(2) XG_PS(3) XG_PS(4) XG_PS(5) XG_PS(6)
 #undef XG_PS
