@@ -319,9 +319,29 @@ void Ensemble::setup() {
   E.ndf = 3;
   E.node_off = d_node_off.p;
   E.ele_off = d_ele_off.p;
-  if (!row_off.empty()) {
-    d_row_off.upload(row_off, s);
-    E.row_off = d_row_off.p;
+  // model of each wavefront item
+  std::vector<int> item_model;
+  E.rows = !row_off.empty() && E.f.rw == 20;
+  for (int k = 0; k < nm; k++) {
+    const int items = E.rows ? row_off[k + 1] - row_off[k] : (ele_off[k + 1] - ele_off[k]) * E.f.nip;
+    item_model.insert(item_model.end(), items, k);
+  }
+  E.nitem = (long long)item_model.size();
+  if (item_model.empty()) item_model.push_back(0);
+  d_item_model.upload(item_model, s);
+  E.item_model = d_item_model.p;
+  d_active.resize(1);
+  d_active.zero(s);
+  E.active = d_active.p;
+  // the largest band (with a vector) that a workgroup's LDS holds; longer
+  // ones are factored in memory
+  E.lds_doubles = 0;
+  int lds_max = 64 << 10;
+  (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, device);
+  lds_max -= 8 << 10;
+  for (int k = 0; k < nm; k++) {
+    const long long q = (long long)(eq_off[k + 1] - eq_off[k]) * (bwv[k] + 2);
+    if (bwv[k] <= 24 && q * 8 <= lds_max) E.lds_doubles = std::max(E.lds_doubles, (int)q);
   }
   E.eq_off = d_eq_off.p;
   E.band_off = d_band_off.p;
@@ -465,6 +485,7 @@ double Ensemble::time_config(int blk, int grd, int reps) {
   XG_HIP(hipEventElapsedTime(&ms, a, b));
   (void)hipEventDestroy(a);
   (void)hipEventDestroy(b);
+  d_active.zero(s);
   status.upload(st, s);
   iter.upload(it, s);
   newton_count.upload(nc, s);

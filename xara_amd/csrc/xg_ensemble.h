@@ -1,6 +1,5 @@
 // Batched ensemble of independent 2D frame models (dispBeamColumn2d over
-// fiber sections) advanced in lock step by Newmark + Newton: one persistent
-// launch per Newton iteration, every workgroup owning whole models.
+// fiber sections) advanced in lock step by Newmark + Newton (xg_ensemble.hip).
 #pragma once
 #include "xg_frame_dev.h"
 
@@ -13,7 +12,12 @@ struct EnsDev {
   // per model (size nmodel or nmodel+1)
   const int* node_off = nullptr;
   const int* ele_off = nullptr;
-  const int* row_off = nullptr;   // first wavefront item of the frame rows (f.rsec), nullptr: none
+  // wavefront items of the fiber update: 20-lane rows (f.rsec) or sections
+  bool rows = false;
+  long long nitem = 0;
+  const int* item_model = nullptr;
+  int lds_doubles = 0;  // LDS of a solving workgroup, for a band and a vector
+  int* active = nullptr;  // models iterating in this step
   const int* eq_off = nullptr;
   const long long* band_off = nullptr;
   const int* bw = nullptr;
