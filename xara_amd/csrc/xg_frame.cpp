@@ -244,35 +244,6 @@ struct FrameGroup : Group {
         nl += nelas_def[df];
         nfib += def_off[df + 1] - def_off[df];
       }
-    // revertToStart states (Steel02.cpp:69-95, Concrete02.cpp:321-337)
-    std::vector<double> stc((size_t)kSteelHist * ns), csc((size_t)kConcHist * nc);
-    std::vector<int> konc(ns, 0);
-    {
-      // steel fibers in pool order
-      for (int e = 0; e < ne; e++)
-        for (int i = 0; i < nip; i++) {
-          const long long sec = (long long)e * nip + i;
-          const int df = secdef[e];
-          for (int fi = def_off[df]; fi < def_off[df + 1]; fi++) {
-            if (fkind[fi] == 1) {
-              const Steel02Param& p = steelp[fmat[fi]];
-              const long long k = sb[sec] + flocal[fi];
-              const double epsy = p.Fy / p.E0;
-              double hist[kSteelHist] = {-epsy, epsy, 0, 0, 0, 0, 0, 0, 0, p.E0};
-              if (p.sigini != 0.0) {
-                hist[7] = p.sigini / p.E0;
-                hist[8] = p.sigini;
-              }
-              for (int c = 0; c < kSteelHist; c++) stc[(size_t)c * ns + k] = hist[c];
-            } else if (fkind[fi] == 2) {
-              const Concrete02Param& p = concp[fmat[fi]];
-              const long long k = cb[sec] + flocal[fi];
-              double hist[kConcHist] = {0, 0, 0, 0, 2.0 * p.fc / p.epsc0};
-              for (int c = 0; c < kConcHist; c++) csc[(size_t)c * nc + k] = hist[c];
-            }
-          }
-        }
-    }
     dconn.upload(conn, s);
     dgeo.upload(geo_h, s);
     dsecdef.upload(secdef, s);
@@ -296,16 +267,13 @@ struct FrameGroup : Group {
     dsteelp.upload(steelp, s);
     dconcp.upload(concp, s);
     delasE.upload(elasE, s);
-    st_c.upload(stc, s);
-    st_t.upload(stc, s);
-    kon_c.upload(konc, s);
-    kon_t.upload(konc, s);
-    cs_c.upload(csc, s);
-    cs_t.upload(csc, s);
-    el_c.resize(std::max(nl, 1LL));
-    el_c.zero(s);
-    el_t.resize(std::max(nl, 1LL));
-    el_t.zero(s);
+    for (DVec<double>* v : {&st_c, &st_t}) v->resize((size_t)kSteelHist * ns);
+    for (DVec<int>* v : {&kon_c, &kon_t}) v->resize(ns);
+    for (DVec<double>* v : {&cs_c, &cs_t}) v->resize((size_t)kConcHist * nc);
+    for (DVec<double>* v : {&el_c, &el_t}) {
+      v->resize(std::max(nl, 1LL));
+      v->zero(s);
+    }
     de.resize((size_t)ord() * nsec);
     de.zero(s);
     ds.resize((size_t)ord() * nsec);
@@ -376,9 +344,7 @@ struct FrameGroup : Group {
       build_rows({0, ne}, s);
     }
     if (force) setup_force(d, def_off, fkind, fmat, fy, fz, fA, GJ, steelp, concp, elasE);
-    stc_init = std::move(stc);
-    csc_init = std::move(csc);
-    konc_init = std::move(konc);
+    launch_frame_start(s, f);
     // Domain::addElement: setDomain + update() at zero displacement
     // (DispBeamColumn2d.cpp:184; ForceBeamColumn2d's first update forms the
     // initial basic stiffness)
@@ -481,8 +447,6 @@ struct FrameGroup : Group {
     for (DVec<double>* v : {&dSe, &dSe_c, &dkv, &dkv_c, &dvprev, &dvprev_c, &dvs, &dvs_c, &dfsec, &dSsr}) v->zero(s);
     dinit.zero(s);
   }
-  std::vector<double> stc_init, csc_init;
-  std::vector<int> konc_init;
 
   // rows of the displacement-based update (section_rows)
   bool rows_on = false;
@@ -585,14 +549,7 @@ struct FrameGroup : Group {
   }
   void revert_to_start(Domain& d) override {
     hipStream_t s = d.stream;
-    st_c.upload(stc_init, s);
-    st_t.upload(stc_init, s);
-    kon_c.upload(konc_init, s);
-    kon_t.upload(konc_init, s);
-    cs_c.upload(csc_init, s);
-    cs_t.upload(csc_init, s);
-    el_c.zero(s);
-    el_t.zero(s);
+    launch_frame_start(s, f);
     if (force) force_zero_state(s);  // ForceBeamColumn2d::revertToStart (:344-376)
     else zero_update(d);
   }

@@ -77,6 +77,7 @@ struct FrameDev {
 };
 
 void launch_frame_update(hipStream_t s, const FrameDev& f, bool d3, const double* U, int* err);
+void launch_frame_start(hipStream_t s, const FrameDev& f);
 void launch_frame_revert(hipStream_t s, const FrameDev& f, bool d3);
 void launch_frame_resid(hipStream_t s, const FrameDev& f, bool d3, double* Re);
 void launch_frame_tangent(hipStream_t s, const FrameDev& f, bool d3, double* Ke);
