@@ -532,7 +532,9 @@ int xg_incr_disp(xg_domain* h, const double* dU) {
 int xg_update(xg_domain* h) {
   return guard([&] {
     auto& d = R(h);
+    XG_HIP(hipEventRecord(d.ev0, d.stream));
     d.update();
+    XG_HIP(hipEventRecord(d.ev1, d.stream));
     XG_HIP(hipStreamSynchronize(d.stream));
     float ms = 0;
     XG_HIP(hipEventElapsedTime(&ms, d.ev0, d.ev1));
@@ -629,7 +631,9 @@ int xg_spmv(xg_domain* h, const double* x, double* y) {
 
 int xg_commit(xg_domain* h) {
   return guard([&] {
-    R(h).commit();
+    auto& d = R(h);
+    d.commit();
+    XG_HIP(hipStreamSynchronize(d.stream));
     return 0;
   });
 }

@@ -224,7 +224,7 @@ struct Domain::TilePlanJob {
 Domain::~Domain() {
   if (tl_job && tl_job->done.valid()) tl_job->done.wait();
   cg_graph_clear();
-  if (tl_read) (void)hipHostFree(tl_read);
+  if (stat_h) (void)hipHostFree(stat_h);
   if (ev0) (void)hipEventDestroy(ev0);
   if (ev1) (void)hipEventDestroy(ev1);
   groups.clear();
@@ -683,14 +683,22 @@ void Domain::setup() {
   q.resize(neq);
   tmpv.resize(neq);
   part.resize(cg_part_size(neq));
-  pcbad.resize(1);
   binv.resize((size_t)neq * ndf);
   bfirst.upload(bf, s);
   bsize.upload(bs, s);
   blk_first.upload(blkf, s);
   blk_size.upload(blks, s);
-  scal.resize(cg_scal_bytes());
-  dscalar.resize(4);
+  if (cg_scal_bytes() > kStCg2 - kStCg) throw Error(XG_ERR_STATE, "status block");
+  stat.resize(kStBytes);
+  stat.zero(s);
+  if (!stat_h) XG_HIP(hipHostMalloc((void**)&stat_h, kStBytes, hipHostMallocDefault));
+  pcbad = (int*)stat.p;
+  pc_diff = pcbad + 1;
+  ctrl = (double*)(stat.p + kStCtrl);
+  dscalar = (double*)(stat.p + kStDot);
+  tl_scal = (TileScal*)(stat.p + kStTile);
+  scal = stat.p + kStCg;
+  scal2 = stat.p + kStCg2;
   for (auto& g : groups) g->setup(*this);
   fused_tangent_tables();
   setup_transient();
@@ -755,10 +763,7 @@ double Domain::ground_accel(double t) const {
 }
 
 void Domain::update() {
-  hipStream_t s = stream;
-  XG_HIP(hipEventRecord(ev0, s));
   for (auto& g : groups) g->update(*this);
-  XG_HIP(hipEventRecord(ev1, s));
   counters.updates++;
   for (auto& g : groups) counters.material_points += g->fibers();
 }
@@ -834,7 +839,7 @@ void Domain::form_tangent() {
 }
 
 Domain::CgBufs Domain::cg_bufs() {
-  return CgBufs{r0.p, r1.p, z.p, p.p, p2.p, q.p, part.p, binv.p, pcbad.p, scal.p, band_A.p, band_L.p, band_Lr.p,
+  return CgBufs{r0.p, r1.p, z.p, p.p, p2.p, q.p, part.p, binv.p, pcbad, scal, band_A.p, band_L.p, band_Lr.p,
                 sw_b.p, sw_x.p, binv_s.p};
 }
 
@@ -853,14 +858,14 @@ void Domain::precond_setup(const CgBufs& w) {
   // the domain's own factor storage (the allocation-free solve's narrow band
   // factor lives in its scratch instead)
   const bool own = (band && w.bandL == band_L.p) || wide;
+  const bool own_flag = w.pcbad == pcbad;
+  XG_HIP(hipMemsetAsync(w.pcbad, 0, own_flag ? 2 * sizeof(int) : sizeof(int), stream));
   if (own && pc_cache && pc_cache_key == key) {
-    XG_HIP(hipMemsetAsync(pc_diff.p, 0, sizeof(int), stream));
-    launch_vals_differ(stream, (long long)num.colind.size(), vals.p, pc_vals.p, pc_diff.p);
-    int diff = 1;
-    XG_HIP(hipMemcpyAsync(&diff, pc_diff.p, sizeof(int), hipMemcpyDeviceToHost, stream));
+    if (!own_flag) XG_HIP(hipMemsetAsync(pc_diff, 0, sizeof(int), stream));
+    launch_vals_differ(stream, (long long)num.colind.size(), vals.p, pc_vals.p, pc_diff);
+    XG_HIP(hipMemcpyAsync(stat_h, stat.p, 2 * sizeof(int), hipMemcpyDeviceToHost, stream));
     XG_HIP(hipStreamSynchronize(stream));
-    if (!diff) {  // the same matrix: its factor is in place (and had no bad pivot)
-      XG_HIP(hipMemsetAsync(w.pcbad, 0, sizeof(int), stream));
+    if (!((const int*)stat_h)[1]) {  // the same matrix: its factor is in place (and had no bad pivot)
       pc_reuses++;
       pc_done = key;
       return;
@@ -871,7 +876,6 @@ void Domain::precond_setup(const CgBufs& w) {
     pc_fresh = pc_reuse_on && pc_vals.n >= num.colind.size();
     pc_fresh_key = key;
   }
-  XG_HIP(hipMemsetAsync(w.pcbad, 0, sizeof(int), stream));
   if (wide) {
     tiles_form(w.pcbad);
   } else if (band) {
@@ -894,7 +898,7 @@ void Domain::tiles_form(int* bad) {
   };
   // plain launches when graphs are off or the flag is not the domain's own
   // (the allocation-free solve: the captured graph is left as it is)
-  if (!cg_graph_on || bad != pcbad.p) {
+  if (!cg_graph_on || bad != pcbad) {
     run();
     return;
   }
@@ -928,27 +932,31 @@ int Domain::solve_wide(int R, const double* const* b, double* const* x, const Cg
   const int n = num.neq;
   const double tol2 = rtol * rtol;
   TilePcg P;
-  P.S = tl_scal.p;
+  P.S = tl_scal;
   P.v[0] = TileRhs{b[0], x[0], w.r0, w.z, w.p, w.q, (int)(warm & 1u)};
   P.v[1] = R > 1 ? TileRhs{b[1], x[1], tl_v.p, tl_v.p + n, tl_v.p + 2 * (size_t)n, tl_v.p + 3 * (size_t)n,
                            (int)(warm >> 1 & 1u)}
                  : P.v[0];
+  bool settled = false;
   auto read = [&] {
-    XG_HIP(hipMemcpyAsync(tl_read, tl_scal.p, R * sizeof(TileScal), hipMemcpyDeviceToHost, stream));
-    XG_HIP(hipStreamSynchronize(stream));
+    read_status(w);
+    if (settled) return 0;
+    settled = true;
+    return precond_settle(w);
   };
+  TileScal* const T = tl_read();
   for (int s = 0; s < R; s++) {
-    tl_read[s].conv = 0;
+    T[s].conv = 0;
     if (P.v[s].warm) spmv(x[s], P.v[s].q, true);
   }
   tiles_pcg_start(stream, n, R, P, tol2);
-  if (warm) read();  // a guess within the tolerance ends its solve before the first iteration
-  for (int it = 0; it < maxit; it++) {
+  int bad = warm ? read() : 0;  // a guess within the tolerance ends its solve before the first iteration
+  for (int it = 0; it < maxit && !bad; it++) {
     const double* rs[2];
     double* zs[2];
     int k = 0;
     for (int s = 0; s < R; s++)
-      if (!tl_read[s].conv) {
+      if (!T[s].conv) {
         rs[k] = P.v[s].r;
         zs[k++] = P.v[s].z;
       }
@@ -956,13 +964,15 @@ int Domain::solve_wide(int R, const double* const* b, double* const* x, const Cg
     tiles_apply(k, rs, zs, graphs);
     tiles_pcg_dir(stream, n, R, P);
     for (int s = 0; s < R; s++)
-      if (!tl_read[s].conv) spmv(P.v[s].p, P.v[s].q, true);
+      if (!T[s].conv) spmv(P.v[s].p, P.v[s].q, true);
     tiles_pcg_step(stream, n, R, P, tol2);
-    read();
+    bad = read();
   }
+  if (!settled) bad = read();
+  if (bad) return bad;
   int status = 0;
   for (int s = 0; s < R; s++) {
-    const TileScal& S = tl_read[s];
+    const TileScal& S = T[s];
     counters.solves++;
     counters.cg_iters += S.iters;
     counters.last_cg_relres = S.bb > 0 ? std::sqrt(S.rr / S.bb) : 0.0;
@@ -1055,8 +1065,6 @@ void Domain::tiles_setup(int bw) {
   tl_Y.resize(2 * np);
   tl_X.resize(2 * np);
   tl_v.resize(4 * (size_t)n);
-  tl_scal.resize(2);
-  if (!tl_read) XG_HIP(hipHostMalloc((void**)&tl_read, 2 * sizeof(TileScal), hipHostMallocDefault));
   tl_bw = bw;
 }
 
@@ -1076,7 +1084,6 @@ void Domain::band_order() {
   tl_factor_us = 0;
   pc_cache = pc_fresh = false;
   pc_vals.release();
-  pc_diff.release();
   band_pinv.release();
   band_A.release();
   band2.release();
@@ -1132,7 +1139,6 @@ void Domain::band_order() {
   band_pinv.upload(pinv, stream);
   band_A.resize((size_t)n * (best + 1));
   band2.resize((size_t)5 * n);
-  scal2.resize(cg_scal_bytes());
   band_L.resize((size_t)n * (best + 1));
   band_Lr.resize((size_t)n * (best + 1));
   pc_buffers();
@@ -1146,7 +1152,6 @@ void Domain::pc_buffers() {
   pc_reuse_on = !(env && env[0] == '0');
   if (!pc_reuse_on) return;
   pc_vals.resize(std::max<size_t>(num.colind.size(), 1));
-  pc_diff.resize(1);
 }
 
 // Destroys the captured chunks once the stream has drained: a replay still
@@ -1212,97 +1217,100 @@ int Domain::solve_pair(const double* b1, double* x1, const double* b2, double* x
   const int n = num.neq;
   if (n > 0 && wide_active()) {
     const CgBufs w = cg_bufs();
-    if (!precond_ready(w)) return XG_BAD_LINEAR_SOLVE;
-    if (wide_active()) {
-      const double* bs[2] = {b1, b2};
-      double* xs[2] = {x1, x2};
-      // the second right-hand side is DisplacementControl's reference load:
-      // its last solution in x2 is the start
-      return solve_wide(2, bs, xs, w, cg_graph_on, (cg_warm_on && dc_hat_valid) ? 2u : 0u);
+    precond_setup(w);
+    const double* bs[2] = {b1, b2};
+    double* xs[2] = {x1, x2};
+    // the second right-hand side is DisplacementControl's reference load:
+    // its last solution in x2 is the start
+    const int r = solve_wide(2, bs, xs, w, cg_graph_on, (cg_warm_on && dc_hat_valid) ? 2u : 0u);
+    if (r <= 0) return r;
+  } else if (n > 0 && band_active() && band2.n >= (size_t)5 * n) {
+    const CgBufs w = cg_bufs();
+    precond_setup(w);
+    const BandRhs R1{b1, x1, w.r0, w.z, w.p, w.q, w.r1, (CGScal*)w.scal};
+    double* v = band2.p;
+    const BandRhs R2{b2, x2, v, v + n, v + 2 * (size_t)n, v + 3 * (size_t)n, v + 4 * (size_t)n, (CGScal*)scal2};
+    cg_solve_band(stream, n, rowptr.p, colind.p, vals.p, band_bw, band_pinv.p, w.bandL, w.bandLr, rtol * rtol, maxit,
+                  w.pcbad, R1, &R2);
+    read_status(w);
+    const int bad = precond_settle(w);
+    if (bad < 0) return XG_BAD_LINEAR_SOLVE;
+    if (bad == 0) {
+      int status = 0;
+      for (int k = 0; k < 2; k++) {
+        int conv = 0, it = 0, brk = 0;
+        double rr = 0, bb = 0;
+        cg_parse_scal(stat_h + (k == 0 ? kStCg : kStCg2), &conv, &it, &rr, &bb, &brk);
+        counters.solves++;
+        counters.cg_iters += it;
+        counters.last_cg_relres = bb > 0 ? std::sqrt(rr / bb) : 0.0;
+        if (bb > 0 && !(rr <= rtol * rtol * bb)) status = XG_BAD_LINEAR_SOLVE;
+      }
+      return status;
     }
-    // the factor gave way to block Jacobi: one solve after the other
-    const int r = solve(b1, x1);
-    return r < 0 ? r : solve(b2, x2);
   }
-  if (n == 0 || !band_active() || band2.n < (size_t)5 * n) {
-    const int r = solve(b1, x1);
-    return r < 0 ? r : solve(b2, x2);
-  }
-  const CgBufs w = cg_bufs();
-  if (!precond_ready(w)) return XG_BAD_LINEAR_SOLVE;
-  if (!band_active()) {  // the factor gave way to the PCG without it
-    const int r = solve(b1, x1);
-    return r < 0 ? r : solve(b2, x2);
-  }
-  const BandRhs R1{b1, x1, w.r0, w.z, w.p, w.q, w.r1, (CGScal*)w.scal};
-  double* v = band2.p;
-  const BandRhs R2{b2, x2, v, v + n, v + 2 * (size_t)n, v + 3 * (size_t)n, v + 4 * (size_t)n, (CGScal*)scal2.p};
-  cg_solve_band(stream, n, rowptr.p, colind.p, vals.p, band_bw, band_pinv.p, w.bandL, w.bandLr, rtol * rtol, maxit,
-                R1, &R2);
-  int bad = 0;
-  XG_HIP(hipMemcpyAsync(&bad, w.pcbad, sizeof(int), hipMemcpyDeviceToHost, stream));
-  int status = 0;
-  for (int k = 0; k < 2; k++) {
-    int conv = 0, it = 0, brk = 0;
-    double rr = 0, bb = 0;
-    cg_read_scal(stream, k == 0 ? w.scal : (void*)scal2.p, &conv, &it, &rr, &bb, &brk);
-    counters.solves++;
-    counters.cg_iters += it;
-    counters.last_cg_relres = bb > 0 ? std::sqrt(rr / bb) : 0.0;
-    if (bb > 0 && !(rr <= rtol * rtol * bb)) status = XG_BAD_LINEAR_SOLVE;
-  }
-  if (bad) return XG_BAD_LINEAR_SOLVE;
-  return status;
+  // no exact factor, or one that gave way to the PCG without it: one solve
+  // after the other
+  const int r = solve(b1, x1);
+  return r < 0 ? r : solve(b2, x2);
 }
 
-// The preconditioner of the current matrix into w, checked: a band factor
-// that met a pivot that is not positive gives way to the PCG without it.
-bool Domain::precond_ready(const CgBufs& w) {
-  for (;;) {
-    const bool exact = band_active() || wide_active();
-    precond_setup(w);
-    int bad = 0;
-    XG_HIP(hipMemcpyAsync(&bad, w.pcbad, sizeof(int), hipMemcpyDeviceToHost, stream));
-    XG_HIP(hipStreamSynchronize(stream));
-    if (!bad) {
-      if (pc_fresh) {  // a factor just formed in the domain's own storage: remember its matrix
-        launch_copy_d(stream, (long long)num.colind.size(), vals.p, pc_vals.p);
-        pc_cache = true;
-        pc_cache_key = pc_fresh_key;
-      }
-      pc_fresh = false;
-      return true;
-    }
-    pc_fresh = false;
-    if (!exact) return false;
-    wb_failed = true;
-    wb_fallbacks++;
-    pc_done = nullptr;
+// The status block to its pinned copy (and a workspace's own flag and
+// scalars in the place of the domain's), waited for.
+void Domain::read_status(const CgBufs& w) {
+  if (pick_on) launch_pick(stream, X.p, dUhat.p, dc_eq, ctrl);
+  XG_HIP(hipMemcpyAsync(stat_h, stat.p, kStBytes, hipMemcpyDeviceToHost, stream));
+  if (w.pcbad != pcbad) {
+    XG_HIP(hipMemcpyAsync(stat_h, w.pcbad, sizeof(int), hipMemcpyDeviceToHost, stream));
+    XG_HIP(hipMemcpyAsync(stat_h + kStCg, w.scal, cg_scal_bytes(), hipMemcpyDeviceToHost, stream));
   }
+  XG_HIP(hipStreamSynchronize(stream));
+}
+
+int Domain::precond_settle(const CgBufs& w) {
+  const bool fresh = pc_fresh;
+  pc_fresh = false;
+  if (!*(const int*)stat_h) {
+    if (fresh) {  // a factor just formed in the domain's own storage: remember its matrix
+      launch_copy_d(stream, (long long)num.colind.size(), vals.p, pc_vals.p);
+      pc_cache = true;
+      pc_cache_key = pc_fresh_key;
+    }
+    return 0;
+  }
+  if (!band_active() && !wide_active()) return -1;
+  wb_failed = true;
+  wb_fallbacks++;
+  pc_done = nullptr;
+  return 1;
 }
 
 int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs, bool warm) {
   const int n = num.neq;
   if (n == 0) return 0;
   const int bw = (system == XG_SYSTEM_PCG_BLOCKJACOBI) ? ndf : 1;
-  if (!precond_ready(w)) return XG_BAD_LINEAR_SOLVE;
+  precond_setup(w);
   int conv = 0, it = 0, brk = 0;
   double rr = 0, bb = 0;
+  int bad = 0;
   if (band_active()) {
     // one workgroup, one launch, preconditioned by the band's exact factor
     const BandRhs R{b, x, w.r0, w.z, w.p, w.q, w.r1, (CGScal*)w.scal, warm ? 1 : 0};
     cg_solve_band(stream, n, rowptr.p, colind.p, vals.p, band_bw, band_pinv.p, w.bandL, w.bandLr, rtol * rtol, maxit,
-                  R);
-    cg_read_scal(stream, w.scal, &conv, &it, &rr, &bb, &brk);
+                  w.pcbad, R);
+    read_status(w);
+    bad = precond_settle(w);
   } else if (wide_active()) {
     const double* bs[1] = {b};
     double* xs[1] = {x};
-    return solve_wide(1, bs, xs, w, graphs, warm ? 1u : 0u);
+    const int r = solve_wide(1, bs, xs, w, graphs, warm ? 1u : 0u);
+    return r > 0 ? solve_with(b, x, w, graphs) : r;
   } else if (small_path()) {
     // the whole solve in one workgroup, one launch
     cg_solve_small(stream, n, (long long)num.colind.size(), rowptr.p, colind.p, vals.p, b, x, bw, w.binv, bfirst.p,
-                   bsize.p, rtol * rtol, maxit, w.scal);
-    cg_read_scal(stream, w.scal, &conv, &it, &rr, &bb, &brk);
+                   bsize.p, rtol * rtol, maxit, w.pcbad, w.scal);
+    read_status(w);
+    bad = precond_settle(w);
   } else {
     // in the sweep order of the symmetric product: b (and a warm start's
     // guess) gathered into it here, the solution scattered back at the end
@@ -1323,8 +1331,10 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
     const int cap = tl_usable() && tl_big() && !tl_on ? tl_cap : INT_MAX;
     const int L = lanes();
     while (true) {
-      cg_read_scal(stream, w.scal, &conv, &it, &rr, &bb, &brk);
-      if (conv) break;
+      read_status(w);
+      if (issued == 0) bad = precond_settle(w);
+      cg_parse_scal(stat_h + kStCg, &conv, &it, &rr, &bb, &brk);
+      if (conv || bad) break;
       // maxit + 1 iterations at most: the fused iteration tests the previous
       // update's convergence at its start, so the last test comes one
       // iteration later (the extra iteration then returns at once, as it
@@ -1344,8 +1354,14 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
       issued += chunk;
       next = std::min(2 * next, 8 * cg_chunk);
     }
-    if (sweep) launch_sweep_perm(stream, sym_view.nbr, sym_view.m, sym_ord.p, w.xs, x, true);
+    if (sweep && !bad) {
+      launch_sweep_perm(stream, sym_view.nbr, sym_view.m, sym_ord.p, w.xs, x, true);
+      if (pick_on) read_status(w);
+    }
   }
+  if (bad < 0) return XG_BAD_LINEAR_SOLVE;
+  if (bad > 0) return solve_with(b, x, w, graphs);  // without the factor, from zero
+  cg_parse_scal(stat_h + kStCg, &conv, &it, &rr, &bb, &brk);
   counters.solves++;
   counters.cg_iters += it;
   counters.last_cg_relres = bb > 0 ? std::sqrt(rr / bb) : 0.0;
@@ -1363,10 +1379,7 @@ void Domain::commit() {
   if (betaKc != 0.0 && Kc.p)
     for (auto& g : groups) g->tangent(*this, Kc.p + g->ke_off);
   for (auto& g : groups) g->commit(*this);
-  Uc.copy_from(U, stream);
-  Vc.copy_from(V, stream);
-  Ac.copy_from(A, stream);
-  XG_HIP(hipStreamSynchronize(stream));
+  launch_copy3(stream, (long long)U.n, U.p, V.p, A.p, Uc.p, Vc.p, Ac.p);
 }
 
 // Domain::revertToLastCommit (Domain.cpp:1925-1939): nodes and elements
@@ -1404,19 +1417,12 @@ void Domain::revert_to_start() {
 }
 
 double Domain::dot_dev(const double* a, const double* b, int n) {
-  launch_dot(stream, n, a, b, part.p, dscalar.p);
-  double h = 0;
-  dscalar.download(&h, 1, stream);
-  return h;
+  launch_dot(stream, n, a, b, part.p, dscalar);
+  XG_HIP(hipMemcpyAsync(stat_h + kStDot, dscalar, sizeof(double), hipMemcpyDeviceToHost, stream));
+  XG_HIP(hipStreamSynchronize(stream));
+  return *(const double*)(stat_h + kStDot);
 }
 double Domain::norm2_dev(const double* v, int n) { return std::sqrt(dot_dev(v, v, n)); }
-double Domain::read_eq(const double* v, int a) {
-  double h = 0;
-  XG_HIP(hipMemcpyAsync(&h, v + a, sizeof(double), hipMemcpyDeviceToHost, stream));
-  XG_HIP(hipStreamSynchronize(stream));
-  return h;
-}
-
 // ---- convergence tests ----------------------------------------------------
 int Domain::run_test(int& iter, std::vector<double>& norms, int& numIncr) {
   double norm;
@@ -1467,15 +1473,16 @@ int Domain::new_step() {
   if (dc_incr < dc_min) dc_incr = dc_min;
   else if (dc_incr > dc_max) dc_incr = dc_max;
   form_tangent();
-  if (solve_from(phat.p, dUhat.p, cg_warm_on && dc_hat_valid) < 0) return XG_BAD_STEP;
+  pick_on = true;
+  const int solved = solve_from(phat.p, dUhat.p, cg_warm_on && dc_hat_valid);
+  pick_on = false;
+  if (solved < 0) return XG_BAD_STEP;
   dc_hat_valid = true;
-  const double dUahat = read_eq(dUhat.p, dc_eq);
+  const double dUahat = ((const double*)(stat_h + kStCtrl))[1];
   if (dUahat == 0.0) return XG_BAD_STEP;
   const double dl = dc_incr / dUahat;
   lambda += dl;
-  XG_HIP(hipMemsetAsync(dU.p, 0, n * sizeof(double), stream));
-  launch_axpby(stream, n, dl, dUhat.p, 0.0, dU.p);
-  incr_disp(dU.p);
+  incr_disp(dUhat.p, dl);
   if (update_checked() < 0) return XG_BAD_STEP;
   dc_last = 0;
   return 0;
@@ -1495,21 +1502,24 @@ int Domain::integ_update(const double* x) {
     return 0;
   }
   // DisplacementControl::update, DisplacementControl.cpp:224-283
-  XG_HIP(hipMemcpyAsync(dUbar.p, x, n * sizeof(double), hipMemcpyDeviceToDevice, stream));
-  const double dUabar = read_eq(dUbar.p, dc_eq);
   const bool hat_ready = dc_hat_ready;
   dc_hat_ready = false;
-  if (!hat_ready && solve_from(phat.p, dUhat.p, cg_warm_on && dc_hat_valid) < 0) return XG_BAD_STEP;
+  if (!hat_ready) {
+    pick_on = true;
+    const int solved = solve_from(phat.p, dUhat.p, cg_warm_on && dc_hat_valid);
+    pick_on = false;
+    if (solved < 0) return XG_BAD_STEP;
+  }
   dc_hat_valid = true;
-  const double dUahat = read_eq(dUhat.p, dc_eq);
+  // the last read_status brought both at the control DOF
+  const double* c = (const double*)(stat_h + kStCtrl);
+  const double dUabar = c[0], dUahat = c[1];
   if (dUahat == 0.0) return XG_BAD_STEP;
   const double dL = -dUabar / dUahat;
-  XG_HIP(hipMemcpyAsync(dU.p, dUbar.p, n * sizeof(double), hipMemcpyDeviceToDevice, stream));
-  launch_axpby(stream, n, dL, dUhat.p, 1.0, dU.p);
+  launch_axpby(stream, n, dL, dUhat.p, 1.0, X.p);
   lambda += dL;
-  incr_disp(dU.p);
+  incr_disp(X.p);
   if (update_checked() < 0) return XG_BAD_STEP;
-  XG_HIP(hipMemcpyAsync(X.p, dU.p, n * sizeof(double), hipMemcpyDeviceToDevice, stream));
   dc_last++;
   return 0;
 }
@@ -1525,7 +1535,10 @@ int Domain::newton() {
     if (integ == 2 && (band_active() || wide_active())) {
       // DisplacementControl::update solves for the reference load with the
       // same matrix: both solves at once
-      if (solve_pair(B.p, X.p, phat.p, dUhat.p) < 0) return XG_BAD_LINEAR_SOLVE;
+      pick_on = true;
+      const int solved = solve_pair(B.p, X.p, phat.p, dUhat.p);
+      pick_on = false;
+      if (solved < 0) return XG_BAD_LINEAR_SOLVE;
       dc_hat_ready = true;
     } else {
       // under LoadControl the first iteration of a step solves for the same
@@ -1568,8 +1581,6 @@ int Domain::analyze(int nsteps, double dtv) {
     dUhat.resize(n);
     dUhat.zero(stream);
     dc_hat_valid = false;
-    dUbar.resize(n);
-    dU.resize(n);
     lambda += 1.0;
     form_unbalance();
     XG_HIP(hipMemcpyAsync(phat.p, B.p, n * sizeof(double), hipMemcpyDeviceToDevice, stream));
@@ -1594,6 +1605,7 @@ int Domain::analyze(int nsteps, double dtv) {
     }
     commit();
   }
+  XG_HIP(hipStreamSynchronize(stream));
   return 0;
 }
 

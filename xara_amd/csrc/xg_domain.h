@@ -125,7 +125,7 @@ struct Domain {
   DVec<double> sw_b, sw_x, binv_s;
   DVec<double> vals, Ke, Re, B, X, Peq;
   DVec<int> asm_ptr, asm_idx, rhs_ptr, rhs_idx;
-  DVec<int> nfail, pcbad;
+  DVec<int> nfail;
   // solver workspace
   DVec<double> r0, r1, z, p, p2, q, part, binv, tmpv;
   DVec<int> bfirst, blk_first;
@@ -137,8 +137,19 @@ struct Domain {
   DVec<unsigned char> fz_a, fz_tgt;
   bool fz_ok = false;
   void fused_tangent_tables();
-  DVec<char> scal;
-  DVec<double> dscalar;
+  // what the host reads between launches, in one device block with a pinned
+  // copy: one transfer and one wait where every flag and scalar had its own
+  static constexpr size_t kStCtrl = 8, kStDot = 24, kStTile = 64, kStCg = 192, kStCg2 = 320, kStBytes = 512;
+  DVec<char> stat;
+  char* stat_h = nullptr;
+  int* pcbad = nullptr;       // the preconditioner met a bad pivot
+  int* pc_diff = nullptr;     // the matrix differs from the last one factored
+  double* ctrl = nullptr;     // DisplacementControl: X and dUhat at the control DOF
+  double* dscalar = nullptr;  // a dot product
+  TileScal* tl_scal = nullptr;
+  char *scal = nullptr, *scal2 = nullptr;  // CGScal of a solve, and of a second one beside it
+  TileScal* tl_read() { return reinterpret_cast<TileScal*>(stat_h + kStTile); }
+  bool pick_on = false;  // read_status also brings ctrl
   int nblk = 0;
   // analysis configuration
   int system = XG_SYSTEM_PCG_JACOBI, numberer = XG_NUMBERER_RCM;
@@ -175,7 +186,7 @@ struct Domain {
   int dc_node = 0, dc_dof = 0, dc_eq = -1;
   double dc_incr = 0, dc_min = 0, dc_max = 0, dc_spec = 1, dc_last = 1;
   bool dc_ready = false;
-  DVec<double> phat, dUhat, dUbar, dU;
+  DVec<double> phat, dUhat;
   double lambda = 0, time = 0, dt = 0;
   // transient (Newmark, UniformExcitation + PathSeries, Rayleigh damping)
   double nm_gamma = 0.5, nm_beta = 0.25, nm_c2 = 0, nm_c3 = 0;
@@ -229,7 +240,6 @@ struct Domain {
   DVec<int> band_pinv;
   DVec<double> band_A, band_L, band_Lr;
   DVec<double> band2;  // work vectors of a second band solve (solve_pair)
-  DVec<char> scal2;
   bool dc_hat_ready = false;  // the Newton iteration has solved for the reference load
   int solve_pair(const double* b1, double* x1, const double* b2, double* x2);
   bool band_active() const { return cg_small_on && band_bw >= 0 && !wb_failed && !wide_active(); }
@@ -268,8 +278,6 @@ struct Domain {
   DVec<int> tl_ints;
   DVec<int4> tl_task;
   DVec<double> tl_A, tl_G, tl_Y, tl_X, tl_v;  // tiles, sweep vectors, 4 PCG vectors of a second right-hand side
-  DVec<TileScal> tl_scal;
-  TileScal* tl_read = nullptr;  // pinned copy of tl_scal
   hipGraph_t tl_fg = nullptr, tl_sg[2] = {nullptr, nullptr};
   hipGraphExec_t tl_fe = nullptr, tl_se[2] = {nullptr, nullptr};
   void tiles_setup(int bw);
@@ -284,7 +292,6 @@ struct Domain {
   // still elastic) keeps its factor instead of being factored again
   // (XG_PC_REUSE=0 turns this off)
   DVec<double> pc_vals;
-  DVec<int> pc_diff;
   bool pc_reuse_on = true, pc_cache = false, pc_fresh = false;
   const void* pc_cache_key = nullptr;
   const void* pc_fresh_key = nullptr;
@@ -294,6 +301,7 @@ struct Domain {
   void pc_buffers();
   void tiles_apply(int k, const double* const* r, double* const* z, bool graphs);
   // warm: bit s set when x[s] holds a guess to start right-hand side s from
+  // 1: the factor met a bad pivot (precond_settle)
   int solve_wide(int R, const double* const* b, double* const* x, const CgBufs& w, bool graphs, unsigned warm = 0);
   // the preconditioner's buffers last formed from the current matrix
   // (nullptr: the matrix changed since), so repeated solves of one matrix
@@ -305,14 +313,16 @@ struct Domain {
   int solve_from(const double* b, double* x, bool warm) { return solve_with(b, x, cg_bufs(), cg_graph_on, warm); }
   // returns < 0 on failure; graphs: replay chunks from captured graphs
   int solve_with(const double* b, double* x, const CgBufs& w, bool graphs, bool warm = false);
-  bool precond_ready(const CgBufs& w);
+  void read_status(const CgBufs& w);
+  // after read_status: 0 the preconditioner is good, 1 an exact factor met a
+  // bad pivot and is dropped (solve again without it), -1 no preconditioner
+  int precond_settle(const CgBufs& w);
   void incr_disp(const double* dU_dev, double scale = 1.0);
-  void commit();
+  void commit();  // queued, like every operation the analysis loop issues
   void revert();
   void revert_to_start();
   double norm2_dev(const double* v, int n);
   double dot_dev(const double* a, const double* b, int n);
-  double read_eq(const double* v, int a);
   int analyze(int nsteps, double dtv);
   long long state_size(int kind);
   void get_state(int kind, double* out);

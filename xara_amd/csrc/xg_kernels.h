@@ -114,6 +114,7 @@ void cg_iterations_check(int bw, const SymSpmv* sym);
 // doubles each
 void band_factor(hipStream_t s, int n, int bw, const int* rowptr, const int* colind, const double* vals,
                  const int* pinv, double* A, double* L, double* Lr, int* bad);
+// (with *bad set, the preconditioner's flag, these two solve nothing)
 // whole band-preconditioned PCG solve in one workgroup per right-hand side
 // (one, or two side by side); r, z, p, q, t: n doubles of work each, S the
 // solve's scalars
@@ -126,14 +127,18 @@ struct BandRhs {
   int warm = 0;  // x holds a guess: start from r = b - A x (stop test unchanged)
 };
 void cg_solve_band(hipStream_t s, int n, const int* rowptr, const int* colind, const double* vals, int bw,
-                   const int* pinv, const double* L, const double* Lr, double tol2, int maxit, const BandRhs& r0,
-                   const BandRhs* r1 = nullptr);
+                   const int* pinv, const double* L, const double* Lr, double tol2, int maxit, const int* bad,
+                   const BandRhs& r0, const BandRhs* r1 = nullptr);
 // whole solve in one workgroup (k_pcg_small) for systems that fit it
 bool cg_small_fits(int n, long long nnz);
 void cg_solve_small(hipStream_t s, int n, long long nnz, const int* rowptr, const int* colind, const double* vals,
                     const double* b, double* x, int bw, const double* binv, const int* bfirst,
-                    const unsigned char* bsize, double tol2, int maxit, void* scal);
-void cg_read_scal(hipStream_t s, const void* scal, int* converged, int* iter, double* rr, double* bb,
-                  int* breakdown);
+                    const unsigned char* bsize, double tol2, int maxit, const int* bad, void* scal);
+// a CGScal copied to the host
+void cg_parse_scal(const void* scal, int* converged, int* iter, double* rr, double* bb, int* breakdown);
+// out[0] = x[i], out[1] = y[i]
+void launch_pick(hipStream_t s, const double* x, const double* y, int i, double* out);
+void launch_copy3(hipStream_t s, long long n, const double* a, const double* b, const double* c, double* x, double* y,
+                  double* z);
 
 }  // namespace xg

@@ -808,7 +808,8 @@ __global__ __launch_bounds__(NT) void k_pcg_small(
     int n, int lg, const int* __restrict__ rowptr, const int* __restrict__ colind, const double* __restrict__ vals,
     const double* __restrict__ b, double* __restrict__ x, const double* __restrict__ binv,
     const int* __restrict__ bfirst, const unsigned char* __restrict__ bsize, double tol2, int maxit,
-    CGScal* __restrict__ S) {
+    const int* __restrict__ bad, CGScal* __restrict__ S) {
+  if (*bad) return;  // no preconditioner: x stays as it is
   __shared__ __align__(16) double shp[NT];
   __shared__ __align__(16) double shr[NT + 8];
   __shared__ __align__(16) double sh[2][2 * kSmallPcgThreads / 64];
@@ -1334,7 +1335,8 @@ __device__ __attribute__((noinline)) void band_sweeps(int n, int bw, const doubl
 __global__ __launch_bounds__(kSmallPcgThreads) void k_pcg_band(
     int n, const int* __restrict__ rowptr, const int* __restrict__ colind, const double* __restrict__ vals, int bw,
     const int* __restrict__ pinv, const double* __restrict__ L, const double* __restrict__ Lr, double tol2, int maxit,
-    BandRhs r0, BandRhs r1) {
+    const int* __restrict__ bad, BandRhs r0, BandRhs r1) {
+  if (*bad) return;  // no factor: x stays as it is
   // workgroup k solves right-hand side k (two independent solves with one
   // factor run side by side on two CUs)
   const BandRhs& R = blockIdx.x == 0 ? r0 : r1;
@@ -1556,6 +1558,20 @@ __global__ __launch_bounds__(128) void k_block_inverse(int nblk, const int* __re
 // ---------------------------------------------------------------------------
 // Small vector kernels
 // ---------------------------------------------------------------------------
+__global__ void k_pick(const double* __restrict__ x, const double* __restrict__ y, int i, double* __restrict__ out) {
+  out[threadIdx.x] = threadIdx.x ? y[i] : x[i];
+}
+
+__global__ void k_copy3(long long n, const double* __restrict__ a, const double* __restrict__ b,
+                        const double* __restrict__ c, double* __restrict__ x, double* __restrict__ y,
+                        double* __restrict__ z) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  x[i] = a[i];
+  y[i] = b[i];
+  z[i] = c[i];
+}
+
 // U[node dof] += dU[eq] over the DOF map (AnalysisModel::incrDisp)
 __global__ void k_incr_disp(long long ndofs, const int* __restrict__ eqmap, const double* __restrict__ dU,
                             double scale, double* __restrict__ U) {
@@ -1777,6 +1793,16 @@ void launch_block_inverse(hipStream_t s, int nblk, const int* first, const unsig
     default: throw Error(XG_ERR_ARG, "block-Jacobi block size must be 1..6");
   }
 }
+void launch_pick(hipStream_t s, const double* x, const double* y, int i, double* out) {
+  hipLaunchKernelGGL(k_pick, dim3(1), dim3(2), 0, s, x, y, i, out);
+}
+
+void launch_copy3(hipStream_t s, long long n, const double* a, const double* b, const double* c, double* x, double* y,
+                  double* z) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_copy3, dim3(ceil_div(n, 256)), dim3(256), 0, s, n, a, b, c, x, y, z);
+}
+
 void launch_incr_disp(hipStream_t s, long long ndofs, const int* eqmap, const double* dU, double scale,
                       double* U) {
   if (ndofs <= 0) return;
@@ -1887,17 +1913,17 @@ void band_factor(hipStream_t s, int n, int bw, const int* rowptr, const int* col
 }
 
 void cg_solve_band(hipStream_t s, int n, const int* rowptr, const int* colind, const double* vals, int bw,
-                   const int* pinv, const double* L, const double* Lr, double tol2, int maxit, const BandRhs& r0,
-                   const BandRhs* r1) {
+                   const int* pinv, const double* L, const double* Lr, double tol2, int maxit, const int* bad,
+                   const BandRhs& r0, const BandRhs* r1) {
   hipLaunchKernelGGL(k_pcg_band, dim3(r1 ? 2 : 1), dim3(kSmallPcgThreads), 0, s, n, rowptr, colind, vals, bw, pinv, L,
-                     Lr, tol2, maxit, r0, r1 ? *r1 : r0);
+                     Lr, tol2, maxit, bad, r0, r1 ? *r1 : r0);
 }
 
 bool cg_small_fits(int n, long long nnz) { return n > 0 && n <= 1024 && nnz <= 32768; }
 
 void cg_solve_small(hipStream_t s, int n, long long nnz, const int* rowptr, const int* colind, const double* vals,
                     const double* b, double* x, int bw, const double* binv, const int* bfirst,
-                    const unsigned char* bsize, double tol2, int maxit, void* scal) {
+                    const unsigned char* bsize, double tol2, int maxit, const int* bad, void* scal) {
   CGScal* S = (CGScal*)scal;
   // lanes per row: twelve entries each, as far as 1,024 threads reach
   int lg = 0;
@@ -1909,10 +1935,10 @@ void cg_solve_small(hipStream_t s, int n, long long nnz, const int* rowptr, cons
   case W:                                                                                                          \
     if (nt <= 768)                                                                                                 \
       hipLaunchKernelGGL((k_pcg_small<W, 768, 44>), g, blk, 0, s, n, lg, rowptr, colind, vals, b, x, binv, bfirst,  \
-                         bsize, tol2, maxit, S);                                                                   \
+                         bsize, tol2, maxit, bad, S);                                                              \
     else                                                                                                           \
       hipLaunchKernelGGL((k_pcg_small<W, 1024, 24>), g, blk, 0, s, n, lg, rowptr, colind, vals, b, x, binv, bfirst, \
-                         bsize, tol2, maxit, S);                                                                   \
+                         bsize, tol2, maxit, bad, S);                                                              \
     break;
     XG_PS(1) XG_PS(2) XG_PS(3) XG_PS(4) XG_PS(5) XG_PS(6)
 #undef XG_PS
@@ -1920,11 +1946,8 @@ void cg_solve_small(hipStream_t s, int n, long long nnz, const int* rowptr, cons
   }
 }
 
-void cg_read_scal(hipStream_t s, const void* scal, int* converged, int* iter, double* rr, double* bb,
-                  int* breakdown) {
-  CGScal h;
-  XG_HIP(hipMemcpyAsync(&h, scal, sizeof(CGScal), hipMemcpyDeviceToHost, s));
-  XG_HIP(hipStreamSynchronize(s));
+void cg_parse_scal(const void* scal, int* converged, int* iter, double* rr, double* bb, int* breakdown) {
+  const CGScal& h = *(const CGScal*)scal;
   *converged = h.converged;
   *iter = std::max(h.iterp[0], h.iterp[1]);
   *rr = h.rr;
