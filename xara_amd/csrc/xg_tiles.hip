@@ -45,12 +45,6 @@ constexpr int SH = HC + 2;  // LDS row stride of a half tile
 
 typedef double d4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ double lane_d(double v, int l) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-  return __hiloint2double(hi, lo);
-}
-
 // 1/a: the hardware estimate and two Newton steps
 __device__ __forceinline__ double rcp_nr(double a) {
   double y = __builtin_amdgcn_rcp(a);
@@ -161,104 +155,154 @@ __device__ __forceinline__ void quad_store(double* __restrict__ g, const d4 (&ac
         g[(32 * (w >> 1) + 16 * a + (l >> 4) + 4 * r) * TB + 32 * (w & 1) + 16 * b + (l & 15)] = acc[a][b][r];
 }
 
-// One pivot (row g0 + C, its column at a[C]) of the symmetric sweep over a
-// panel of PW columns, lane r holding row r of the panel: every other row
-// takes its multiple of the pivot row off, the pivot row is left unscaled
-// (its lane multiplies it by 1/pivot after the panel, which commutes with
-// the later row operations).
+// The value of lane C of the lane's row of 16
 template <int C>
-__device__ __forceinline__ void sweep_pivot(double (&a)[PW], double& scale, int g0, bool& nonpos) {
-  const int l = threadIdx.x & 63, g = g0 + C;
-  double row[PW];
-#pragma unroll
-  for (int j = 0; j < PW; j++) row[j] = lane_d(a[j], g);
-  // not positive (or not a number): the caller drops the whole factor, so
-  // what follows from it does not matter
-  nonpos |= !(row[C] > 0.0) || !isfinite(row[C]);
-  const double inv = rcp_nr(row[C]);
-  const bool own = l == g;
+__device__ __forceinline__ double row_d(double v) {
+  const long long b = __double_as_longlong(v);
+  return __longlong_as_double(__builtin_amdgcn_update_dpp(b, b, 0x150 + C, 0xf, 0xf, true));
+}
+
+// One pivot (row g0 + C, in lane C of every 16, its column at a[C]) of the
+// symmetric sweep over a panel of PW columns, the lane holding row `row` of
+// the panel: every other row takes its multiple of the pivot row off, the
+// pivot row is left unscaled (its lane multiplies it by 1/pivot after the
+// panel, which commutes with the later row operations).
+template <int C>
+__device__ __forceinline__ void sweep_pivot(double (&a)[PW], double& scale, int row, int g0) {
+  const double inv = rcp_nr(row_d<C>(a[C]));
+  const bool own = row == g0 + C;
   const double u = own ? 0.0 : a[C] * inv;
   if (own) scale = inv;
 #pragma unroll
   for (int j = 0; j < PW; j++)
-    if (j != C) a[j] = fma(-u, row[j], a[j]);
-  a[C] = own ? -1.0 : u;
+    if (j != C) a[j] = fma(-u, row_d<C>(a[j]), a[j]);
+  // (u is 0 in the pivot's own lane: one half of -1)
+  a[C] = __hiloint2double(own ? 0xbff00000 : __double2hiint(u), __double2loint(u));
 }
 
+// What a panel leaves to be done after the next barrier: the products of
+// blocks 1 .. 3 (as numbered then), A operand a, B operands b
+struct Pending {
+  double a[2], b[3][2];
+};
+
 // One panel, columns 16 p + 8 H .., of the symmetric sweep: m[J] the block
-// (w, (p + J) % 4) of the wavefront's block row.
+// (w, (p + J) % 4) of the wavefront's block row.  P holds the panel's
+// columns, Wp the last panel as swept, W takes this one, Pn the next panel.
 template <int H>
-__device__ __forceinline__ void panel_step(d4 (&m)[4], double* P, double* W, int p, int w, bool& nonpos) {
+__device__ __forceinline__ void panel_step(d4 (&m)[4], double* P, double* Pn, double* W, const double* Wp, int p,
+                                           int w, bool& nonpos, Pending& q) {
+  constexpr int HP = 1 - H, E = H;  // E: the block that holds the next panel
   const int l = threadIdx.x & 63, lc = l & 15, lr = l >> 4;
-  const bool mine = (lc >> 3) == H;
-  if (mine)
-#pragma unroll
-    for (int r = 0; r < 4; r++) P[(16 * w + lr + 4 * r) * SP + (lc & 7)] = m[0][r];
+  const int g0 = 16 * p + 8 * H, row = lc < 8 ? g0 + lc : 16 * w + 8 * (lr & 1) + lc - 8;
   __syncthreads();
-  double a[PW];
+  double a[PW], v[4][2], vm[4], b[4][2];
 #pragma unroll
   for (int j = 0; j < PW; j += 2) {
-    const double2 v = *reinterpret_cast<const double2*>(P + l * SP + j);
-    a[j] = v.x;
-    a[j + 1] = v.y;
+    const double2 x = *reinterpret_cast<const double2*>(P + row * SP + j);
+    a[j] = x.x;
+    a[j + 1] = x.y;
   }
-  double scale = 1.0;
-  const int g0 = 16 * p + 8 * H;
-  sweep_pivot<0>(a, scale, g0, nonpos);
-  sweep_pivot<1>(a, scale, g0, nonpos);
-  sweep_pivot<2>(a, scale, g0, nonpos);
-  sweep_pivot<3>(a, scale, g0, nonpos);
-  sweep_pivot<4>(a, scale, g0, nonpos);
-  sweep_pivot<5>(a, scale, g0, nonpos);
-  sweep_pivot<6>(a, scale, g0, nonpos);
-  sweep_pivot<7>(a, scale, g0, nonpos);
-#pragma unroll
-  for (int j = 0; j < PW; j += 2)
-    *reinterpret_cast<double2*>(W + l * SP + j) = make_double2(a[j] * scale, a[j + 1] * scale);
-  wave_order();
-  // the rest of the matrix: block (I, J) -= W_I P_J^T; the swept columns and
-  // rows (registers 2 H and 2 H + 1 of block row p) then taken from W
-  const double a0 = -W[(16 * w + lc) * SP + lr], a1 = -W[(16 * w + lc) * SP + 4 + lr];
-  const bool prow = w == p;
 #pragma unroll
   for (int J = 0; J < 4; J++) {
     const int c = (16 * ((p + J) & 3) + lc) * SP + lr;
-    m[J] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, P[c], m[J], 0, 0, 0);
-    m[J] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, P[c + 4], m[J], 0, 0, 0);
-    const double v0 = W[c], v1 = W[c + 4];
-    if (J == 0) {
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const double v = W[(16 * w + lr + 4 * r) * SP + (lc & 7)];
-        m[0][r] = mine ? v : m[0][r];
-      }
-    }
-    m[J][2 * H] = prow ? v0 : m[J][2 * H];
-    m[J][2 * H + 1] = prow ? v1 : m[J][2 * H + 1];
+    v[J][0] = Wp[c];
+    v[J][1] = Wp[c + 4];
+    b[J][0] = P[c];
+    b[J][1] = P[c + 4];
   }
+  if (H == 0)
+#pragma unroll
+    for (int r = 0; r < 4; r++) vm[r] = Wp[(16 * w + lr + 4 * r) * SP + (lc & 7)];
+  // the last panel's products, while this one comes from LDS
+#pragma unroll
+  for (int k = 0; k < 2; k++)
+#pragma unroll
+    for (int J = 1; J < 4; J++) m[J] = __builtin_amdgcn_mfma_f64_16x16x4f64(q.a[k], q.b[J - 1][k], m[J], 0, 0, 0);
+  double scale = 1.0;
+  sweep_pivot<0>(a, scale, row, g0);
+  sweep_pivot<1>(a, scale, row, g0);
+  sweep_pivot<2>(a, scale, row, g0);
+  sweep_pivot<3>(a, scale, row, g0);
+  sweep_pivot<4>(a, scale, row, g0);
+  sweep_pivot<5>(a, scale, row, g0);
+  sweep_pivot<6>(a, scale, row, g0);
+  sweep_pivot<7>(a, scale, row, g0);
+  // the last panel's columns and rows (registers 2 HP and 2 HP + 1 of its
+  // block row) from the panel as swept; the next panel's block had its
+  // columns, and for H = 1 its rows, before
+  if (H == 0) {
+    const bool swept = p > 0 && (lc >> 3) == HP;
+#pragma unroll
+    for (int r = 0; r < 4; r++) m[3][r] = swept ? vm[r] : m[3][r];
+  }
+  const bool prow = w == (H == 0 ? p - 1 : p);
+#pragma unroll
+  for (int J = H == 0 ? 0 : 1; J < 4; J++) {
+    m[J][2 * HP] = prow ? v[J][0] : m[J][2 * HP];
+    m[J][2 * HP + 1] = prow ? v[J][1] : m[J][2 * HP + 1];
+  }
+  // a pivot that is not positive (or not a number): the caller drops the
+  // whole factor, so what follows from it does not matter
+  nonpos |= !(scale > 0.0) || !isfinite(scale);
+  if (lc >= 8 && lr < 2)
+#pragma unroll
+    for (int j = 0; j < PW; j += 2)
+      *reinterpret_cast<double2*>(W + row * SP + j) = make_double2(a[j] * scale, a[j + 1] * scale);
   wave_order();
+  // block (I, J) -= W_I P_J^T: the next panel's now
+  q.a[0] = -W[(16 * w + lc) * SP + lr];
+  q.a[1] = -W[(16 * w + lc) * SP + 4 + lr];
+  m[E] = __builtin_amdgcn_mfma_f64_16x16x4f64(q.a[0], b[E][0], m[E], 0, 0, 0);
+  m[E] = __builtin_amdgcn_mfma_f64_16x16x4f64(q.a[1], b[E][1], m[E], 0, 0, 0);
+#pragma unroll
+  for (int J = 1; J < 4; J++)
+#pragma unroll
+    for (int k = 0; k < 2; k++) q.b[J - 1][k] = b[(J + E) & 3][k];
+  if (H == 0) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const double x = W[(16 * w + lr + 4 * r) * SP + (lc & 7)];
+      m[0][r] = lc < 8 ? x : m[0][r];
+    }
+    m[0][0] = w == p ? -q.a[0] : m[0][0];
+    m[0][1] = w == p ? -q.a[1] : m[0][1];
+    if (lc >= 8)
+#pragma unroll
+      for (int r = 0; r < 4; r++) Pn[(16 * w + lr + 4 * r) * SP + lc - 8] = m[0][r];
+  } else {
+    // this panel's rows of the next, from the wavefront that swept them as
+    // its columns
+    if (lc < 8)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        if (r < 2 || w != p) Pn[(16 * w + lr + 4 * r) * SP + lc] = m[1][r];
+    if (w == ((p + 1) & 3)) Pn[(16 * p + 8 + (l >> 3)) * SP + (l & 7)] = W[(16 * w + (l & 7)) * SP + (l >> 3)];
+  }
 }
 
 // Task {column k, first row tile, row tiles} of a level: the inverse of the
 // diagonal block, in every workgroup of the column, by the symmetric sweep
 // in panels of 8 columns (wavefront w keeps block row w of 16 x 16 blocks in
-// accumulators; every wavefront sweeps the panel itself, so one barrier per
-// panel), then G(i, k) = A(i, k) D_k for its row tiles.  The first workgroup
-// of a column stores D_k.
+// accumulators and sweeps its 16 rows of the panel, the 8 pivot rows beside
+// them in every 16 lanes, so one barrier per panel), then G(i, k) = A(i, k)
+// D_k for its row tiles.  The first workgroup of a column stores D_k.
 //
-// Bound by the pivots' chain (224 cycles each, in 64 x 224 of the 33,000
-// cycles of the sweep; the rest the update after each panel): a pivot row
-// reaches the other lanes through readlane, two per column of the panel.
-// Panels of 8 balance that against the matrix-core updates (of 16: 413
-// cycles a pivot).  One column with one row tile, launch to launch: 19.2 us
-// (24.9 with panels of 16; the 4 x 4 register-blocked band factor that this
-// kernel replaces took 41 per tile column).
+// Bound by the pivots' chain and the passage of a panel through LDS.  A
+// pivot row reaches the other lanes by one DPP move a value, and of the
+// products after a panel only the next panel's block is waited for; the
+// others fill the wait for its columns.  Of the 24,100 cycles of the sweep
+// 141 go to each of 64 pivots.  Panels of 8 balance the pivots against the
+// products.  One column with one row tile, launch to launch: 15.7 us (19.2
+// when every wavefront swept all 64 rows, pivot rows by readlane, 224 cycles
+// a pivot, with all products before the next panel; 16.1 with the products
+// held between the pivots; the 4 x 4 register-blocked band factor before
+// took 41 per tile column).
 __global__ __launch_bounds__(256) void k_tl_panel(TileView V, const int4* __restrict__ task,
                                                   const double* __restrict__ A, double* __restrict__ G,
                                                   int* __restrict__ bad) {
   __shared__ __align__(16) double sh[2 * TB * SK];
-  double* pan = sh;                   // two panels, 64 x SP
-  double* wp = sh + 2 * TB * SP;      // a swept panel per wavefront
+  double *P0 = sh, *P1 = sh + TB * SP, *W0 = sh + 2 * TB * SP, *W1 = sh + 3 * TB * SP;
   const int4 t = task[blockIdx.x];
   // the wavefront's number as a scalar: matrix instructions ignore the lane
   // mask, so the branch on it has to be a jump
@@ -276,23 +320,45 @@ __global__ __launch_bounds__(256) void k_tl_panel(TileView V, const int4* __rest
   double2 x[8];
   if (t.z > 0) tile_get(x, A + (dslot + 1 + t.y) * TS, 16 * np);
   bool nonpos = false;
-  double* W = wp + w * TB * SP;
   const int lc = l & 15, lr = l >> 4;
+  if (lc < 8)
+#pragma unroll
+    for (int r = 0; r < 4; r++) P0[(16 * w + lr + 4 * r) * SP + lc] = m[0][r];
+  Pending q = {};
   // the block column in work is m[0]: after each one the blocks move round
   // by one, and everything in the loop is straight-line code (branches on
   // the block column made the compiler copy all accumulators at every one:
   // 42 us)
 #pragma unroll 1
   for (int p = 0; p < np; p++) {
-    panel_step<0>(m, pan, W, p, w, nonpos);
-    panel_step<1>(m, pan + TB * SP, W, p, w, nonpos);
+    panel_step<0>(m, P0, P1, W0, W1, p, w, nonpos, q);
+    panel_step<1>(m, P1, P0, W1, W0, p, w, nonpos, q);
     const d4 m0 = m[0];
     m[0] = m[1];
     m[1] = m[2];
     m[2] = m[3];
     m[3] = m0;
   }
-  if (nonpos && t.y == 0 && threadIdx.x == 0) atomicExch(bad, 1);
+  // what the last panel left
+  __syncthreads();
+#pragma unroll
+  for (int J = 0; J < 4; J++) {
+    if (J > 0) {
+      m[J] = __builtin_amdgcn_mfma_f64_16x16x4f64(q.a[0], q.b[J > 0 ? J - 1 : 0][0], m[J], 0, 0, 0);
+      m[J] = __builtin_amdgcn_mfma_f64_16x16x4f64(q.a[1], q.b[J > 0 ? J - 1 : 0][1], m[J], 0, 0, 0);
+    }
+    const int c = (16 * ((np + J) & 3) + lc) * SP + lr;
+    if (J == 3)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const double v = W1[(16 * w + lr + 4 * r) * SP + (lc & 7)];
+        m[3][r] = lc >= 8 ? v : m[3][r];
+      }
+    const double v0 = W1[c], v1 = W1[c + 4];
+    m[J][2] = w == np - 1 ? v0 : m[J][2];
+    m[J][3] = w == np - 1 ? v1 : m[J][3];
+  }
+  if (nonpos && t.y == 0 && w == 0) atomicExch(bad, 1);
   __syncthreads();
   // D = -m, zero outside the column's panels
   double* X = sh;
