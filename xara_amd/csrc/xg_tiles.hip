@@ -440,6 +440,58 @@ __global__ __launch_bounds__(256) void k_tl_update(const int* __restrict__ tgt, 
   quad_store(T, acc);
 }
 
+// The same for a quarter of the target, four workgroups to a tile, whole
+// sources staged: for levels with too few targets to fill the chip, where
+// the products of one tile follow each other in one compute unit.
+__device__ __forceinline__ void quarter_get(double2 (&v)[4], const double* __restrict__ g, int kc) {
+  const int c = 2 * (threadIdx.x % 32), r = threadIdx.x / 32;
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    v[i] = c < kc ? *reinterpret_cast<const double2*>(g + (r + 8 * i) * TB + c) : make_double2(0.0, 0.0);
+}
+__device__ __forceinline__ void quarter_put(double* s, const double2 (&v)[4]) {
+  const int c = 2 * (threadIdx.x % 32), r = threadIdx.x / 32;
+#pragma unroll
+  for (int i = 0; i < 4; i++) *reinterpret_cast<double2*>(s + (r + 8 * i) * SK + c) = v[i];
+}
+__global__ __launch_bounds__(256) void k_tl_update_quarter(const int* __restrict__ tgt, const int* __restrict__ src,
+                                                           const int* __restrict__ sg, const int* __restrict__ sa,
+                                                           const int* __restrict__ sk, double* __restrict__ A,
+                                                           const double* __restrict__ G) {
+  __shared__ __align__(16) double X[TB / 2 * SK];
+  __shared__ __align__(16) double Y[TB / 2 * SK];
+  const int t = blockIdx.x >> 2, row = 32 * (blockIdx.x >> 1 & 1), col = 32 * (blockIdx.x & 1);
+  const int b = src[t], e = src[t + 1], l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  double* T = A + (long long)tgt[t] * TS + (row + 16 * (w >> 1) + (l >> 4)) * TB + col + 16 * (w & 1) + (l & 15);
+  const double* x0 = X + (16 * (w >> 1) + (l & 15)) * SK + (l >> 4);
+  const double* y0 = Y + (16 * (w & 1) + (l & 15)) * SK + (l >> 4);
+  double2 x[4], y[4];
+  int kc = sk[b];
+  quarter_get(x, G + (long long)sg[b] * TS + row * TB, kc);
+  quarter_get(y, A + (long long)sa[b] * TS + col * TB, kc);
+  d4 acc;
+#pragma unroll
+  for (int r = 0; r < 4; r++) acc[r] = T[4 * r * TB];
+  for (int s = b; s < e; s++) {
+    quarter_put(X, x);
+    quarter_put(Y, y);
+    __syncthreads();
+    const int now = kc;
+    if (s + 1 < e) {
+      kc = sk[s + 1];
+      quarter_get(x, G + (long long)sg[s + 1] * TS + row * TB, kc);
+      quarter_get(y, A + (long long)sa[s + 1] * TS + col * TB, kc);
+    }
+    for (int k = 0; k < now; k += 16)
+#pragma unroll
+      for (int i = 0; i < 16; i += 4)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-x0[k + i], y0[k + i], acc, 0, 0, 0);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++) T[4 * r * TB] = acc[r];
+}
+
 // Sweeps: 1,024 threads per row tile (forward) or column (backward).
 // Forward: four sources at a time, 256 threads each (row t / 4, columns
 // 16 (t % 4) ..), the partial sums added in order.
@@ -652,6 +704,13 @@ __global__ __launch_bounds__(1024) void k_tl_step(int n, TilePcg P, double tol2)
 
 }  // namespace
 
+// Levels of up to this many targets are updated in quarter tiles.  Above it
+// the chip is full and whole tiles read half as much: 33^3 bricks, levels of
+// up to thousands, 137 ms a pass with the line at 512 or 1,024, 145 with
+// quarters throughout.  Below it quarters win: 10 x 10 x 20 frame 21.0 ms
+// without them, 20.1 with the line at 256, 19.4 at 1,024; 12^3 bricks 6.5,
+// 5.9, 5.7; 64 x 16 quad mesh 7.1, 6.4 (a tile of four sources 10.6 -> 8 us).
+constexpr int kTileSplit = 1024;
 void tiles_factor(hipStream_t s, int n, const TileView& V, const TileHost& H, const int* rowptr, const int* colind,
                   const double* vals, double* A, double* G, int* bad) {
   if (n <= 0) return;
@@ -664,9 +723,12 @@ void tiles_factor(hipStream_t s, int n, const TileView& V, const TileHost& H, co
     hipLaunchKernelGGL(k_tl_panel, dim3(H.panptr[l + 1] - H.panptr[l]), dim3(256), 0, s, V, V.task + H.panptr[l], A, G,
                        bad);
     const int nu = H.upptr[l + 1] - H.upptr[l];
-    if (nu > 0)
+    if (nu > kTileSplit)
       hipLaunchKernelGGL(k_tl_update, dim3(nu), dim3(256), 0, s, V.uptgt + H.upptr[l], V.upsrc + H.upptr[l], V.srcg,
                          V.srca, V.srck, A, G);
+    else if (nu > 0)
+      hipLaunchKernelGGL(k_tl_update_quarter, dim3(4 * nu), dim3(256), 0, s, V.uptgt + H.upptr[l],
+                         V.upsrc + H.upptr[l], V.srcg, V.srca, V.srck, A, G);
   }
 }
 
