@@ -207,7 +207,10 @@ int  xg_spmv_config(xg_domain* d, int format, int lanes);
                           equations are preconditioned by their exact tiled
                           sparse factor in nested-dissection order (one or
                           two PCG iterations per solve) where it fits in
-                          2 x 1 GiB; on by default                          */
+                          2 x 4 GiB; a factor estimated above 3 ms is first
+                          formed when a solve without it has cost as much,
+                          and used from then on until revertToStart; on by
+                          default                                           */
 int  xg_cg_config(xg_domain* d, int chunk, int flags);
 /* `numberer RCM|Plain`                                                       */
 int  xg_numberer(xg_domain* d, int kind);
