@@ -310,7 +310,7 @@ int  xg_time_op(xg_domain* d, int op, int reps, double* ms);
    dispBeamColumn over fiber sections, nodal masses, UniformExcitation,
    Newmark, NormDispIncr/NormUnbalance test) whose `analyze n dt` would run
    BasicAnalysisBuilder::analyzeTransient (BasicAnalysisBuilder.cpp:422-520).
-   All members advance together: one persistent launch per Newton iteration,
+   All members advance together: three launches per Newton iteration,
    one captured hipGraph per time step.  A member whose step fails is
    reverted to its last committed state and stops, as its analyze would. */
 typedef struct xg_ensemble xg_ensemble;

@@ -3,8 +3,8 @@
 Each member is an ordinary ``Model`` (2D dispBeamColumn frame with fiber
 sections, nodal masses, UniformExcitation, Newmark, NormDispIncr test)
 defined through the usual commands; ``Ensemble.add`` snapshots its
-definition.  ``analyze`` advances every member by Newmark steps with one
-persistent launch per Newton iteration, captured as one hipGraph per step.
+definition.  ``analyze`` advances every member by Newmark steps with three
+launches per Newton iteration, captured as one hipGraph per step.
 """
 import ctypes as C
 
