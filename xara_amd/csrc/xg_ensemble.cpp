@@ -339,6 +339,12 @@ void Ensemble::setup() {
   int lds_max = 64 << 10;
   (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, device);
   lds_max -= 8 << 10;
+  // with more than four members to a compute unit, four workgroups have to
+  // fit its 160 KB side by side: 4,096 frames 116.3 thousand model-steps/s
+  // with bands up to 38 KB in LDS, 111.2 with those up to 56 KB
+  int cus = 256;
+  (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
+  if (nm > 4 * cus) lds_max = std::min(lds_max, 38 << 10);
   for (int k = 0; k < nm; k++) {
     const long long q = (long long)(eq_off[k + 1] - eq_off[k]) * (bwv[k] + 2);
     if (bwv[k] <= 24 && q * 8 <= lds_max) E.lds_doubles = std::max(E.lds_doubles, (int)q);
