@@ -3,12 +3,15 @@ CPU oracle's direct solve, at the edges of its sizes: the fewest equations
 it takes, columns of 1 to 64 equations, one to many levels, DOFs fixed inside
 the model, 1 to many sources per update; single solves, the allocation-free
 solve bit for bit, and the paired solves of DisplacementControl."""
+import os
+import time
+
 import numpy as np
 import pytest
 
 from tests import _oracle
 from xara_amd import _lib, meshes
-from xara_amd.model import Model
+from xara_amd.model import Model, XaraError
 
 pytestmark = pytest.mark.gpu
 EPS = np.finfo(float).eps
@@ -139,3 +142,38 @@ def test_large_solid_goes_on_with_the_factor():
     (a, ia), (b, ib), (c, ic) = runs
     assert relerr(a, c) <= 1e-9 and relerr(b, c) <= 1e-9
     assert ia < 0.8 * ic and ib < 0.8 * ic
+
+
+def test_failed_setup_leaves_no_thread():
+    """The plan is built on a thread beside the set-up and reads the model's
+    numbering and coordinates: a set-up that fails (here on an element of no
+    length, while the plan of 40,000 loose nodes is being built) returns with
+    that thread ended, and the corrected model is set up as a fresh one is."""
+    print("case: failed set-up with 40,000 loose nodes", flush=True)
+    fr = meshes.rc_frame_3d(3, 3, 6)
+    fresh, m = Model(3, 6), Model(3, 6)
+    for g in (fresh, m):
+        meshes.build_rc_frame_3d(g, fr)
+    fresh.setup()  # the runtime's own threads exist from here on
+    loose = np.arange(10**6, 10**6 + 40000, dtype=np.int32)
+    m.nodes(loose, np.random.default_rng(1).uniform(0, 1e4, (len(loose), 3)))
+    below, top = (int(np.flatnonzero(fr["node_tags"] == t)[0]) for t in fr["columns"][-1])
+    tag = fr["node_tags"][top:top + 1]
+    m.nodes(tag, fr["crds"][below:below + 1])
+    for _ in range(2):
+        before = set(os.listdir("/proc/self/task"))
+        with pytest.raises(XaraError, match="zero length"):
+            m.setup()
+        time.sleep(0.005)  # a joined thread's entry goes a moment later
+        assert set(os.listdir("/proc/self/task")) <= before
+    m.nodes(tag, fr["crds"][top:top + 1])
+    m.fix_many(loose, np.ones((len(loose), 6), np.int32))
+    m.setup()
+    B = np.random.default_rng(0).normal(size=m.neq)
+    X = []
+    for g in (m, fresh):
+        g.form_tangent(values=False)
+        X.append(g.solve(B))
+        assert g.counters()["band_bw"] > 0
+        g.close()
+    assert np.array_equal(*X)

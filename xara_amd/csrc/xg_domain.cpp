@@ -216,13 +216,14 @@ struct J2Group : Group {
 // ---------------------------------------------------------------------------
 // Domain
 // ---------------------------------------------------------------------------
+// A local of setup(): `done` is destroyed first, which waits for the thread,
+// so no set-up leaves one behind, also when it throws.
 struct Domain::TilePlanJob {
   TilePlan plan;
   std::future<bool> done;
 };
 
 Domain::~Domain() {
-  if (tl_job && tl_job->done.valid()) tl_job->done.wait();
   cg_graph_clear();
   if (stat_h) (void)hipHostFree(stat_h);
   if (ev0) (void)hipEventDestroy(ev0);
@@ -536,7 +537,8 @@ void Domain::setup() {
   number_and_pattern(nnode, ndf, fixed, elem_nodes, numberer == XG_NUMBERER_RCM, num);
   const int neq = num.neq;
   const long long nnz = (long long)num.colind.size();
-  tiles_plan_start();
+  TilePlanJob plan;
+  tiles_plan_start(plan);
   // element matrix / vector offsets
   ke_total = re_total = 0;
   for (auto& g : groups) {
@@ -705,7 +707,7 @@ void Domain::setup() {
   // the PCG's block-symmetric layout depends only on the pattern: built here
   // with the other index maps rather than in the first solve
   if (spmv_format != XG_SPMV_CSR) sym_prepare(true);
-  band_order();
+  band_order(plan);
   pc_done = nullptr;
   wb_failed = false;
   XG_HIP(hipStreamSynchronize(s));
@@ -983,33 +985,26 @@ int Domain::solve_wide(int R, const double* const* b, double* const* x, const Cg
 
 // Starts the tiled factorisation's plan (host code) on a thread of its own:
 // it reads the numbering and the coordinates, which the rest of the set-up
-// leaves alone.  Without a thread to spare it runs here.
-void Domain::tiles_plan_start() {
-  if (tl_job && tl_job->done.valid()) tl_job->done.wait();  // of a set-up that threw
-  tl_job.reset();
+// leaves alone.  Without a thread to spare it runs in tiles_setup().
+void Domain::tiles_plan_start(TilePlanJob& job) {
   const int n = num.neq;
   if (n < kTileMinEqn || n > kTileMaxEqn) return;
-  tl_job = std::make_shared<TilePlanJob>();
-  TilePlanJob* job = tl_job.get();
-  auto build = [this, n, job] {
+  auto build = [this, n, &job] {
     const long long max_tiles = (long long)(kTileMaxBytes / (sizeof(double) * kTile * kTile));
-    return tile_plan(n, num.rowptr, num.colind, nnode, ndf, ndm, num.eq, crd_h, max_tiles, 1e300, job->plan);
+    return tile_plan(n, num.rowptr, num.colind, nnode, ndf, ndm, num.eq, crd_h, max_tiles, 1e300, job.plan);
   };
   try {
-    job->done = std::async(std::launch::async, build);
+    job.done = std::async(std::launch::async, build);
   } catch (const std::system_error&) {
-    job->done = std::async(std::launch::deferred, build);
+    job.done = std::async(std::launch::deferred, build);
   }
 }
 
 // Takes the system into the tiled factorisation where its plan fits: the
 // device arrays of its launches.
-void Domain::tiles_setup(int bw) {
-  if (!tl_job) return;
-  const bool ok = tl_job->done.get();
-  const TilePlan P = std::move(tl_job->plan);
-  tl_job.reset();
-  if (!ok) return;
+void Domain::tiles_setup(TilePlanJob& job, int bw) {
+  if (!job.done.valid() || !job.done.get()) return;
+  const TilePlan& P = job.plan;
   const int n = num.neq;
   tl_factor_us = 25.0 * P.nlev + P.flops / 30e6;
   tl_iter_us = 15.0 + 0.55 * 8.0 * (double)num.colind.size() / 3.4e6;
@@ -1078,7 +1073,7 @@ static int band_width(const Numbering& num, const std::vector<int>& pinv) {
   return bw;
 }
 
-void Domain::band_order() {
+void Domain::band_order(TilePlanJob& plan) {
   band_bw = -1;
   tl_bw = -1;
   tl_factor_us = 0;
@@ -1132,7 +1127,7 @@ void Domain::band_order() {
       pinv = geo;
     }
   }
-  tiles_setup(best);
+  tiles_setup(plan, best);
   if (tl_bw >= 0) pc_buffers();
   if (best > 63 || n > kBandMaxEqn) return;
   band_bw = best;

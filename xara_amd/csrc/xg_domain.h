@@ -243,7 +243,8 @@ struct Domain {
   bool dc_hat_ready = false;  // the Newton iteration has solved for the reference load
   int solve_pair(const double* b1, double* x1, const double* b2, double* x2);
   bool band_active() const { return cg_small_on && band_bw >= 0 && !wb_failed && !wide_active(); }
-  void band_order();
+  struct TilePlanJob;  // the tiled factor's plan, built on a thread beside the rest of the set-up
+  void band_order(TilePlanJob& plan);
   // tiled sparse factorisation (xg_tiles.hip), the exact preconditioner
   // under the static integrators of the systems tiles_setup() takes (a
   // transient's K + c3 M is well conditioned by the mass term: block Jacobi
@@ -268,10 +269,7 @@ struct Domain {
   int tl_cap = 0;
   bool tl_big() const { return tl_factor_us > kTileBigUs; }
   bool tl_usable() const { return cg_small_on && cg_wide_on && !wb_failed && tl_bw >= 0 && integ != 3; }
-  // the plan, built beside the rest of the set-up
-  struct TilePlanJob;
-  std::shared_ptr<TilePlanJob> tl_job;
-  void tiles_plan_start();
+  void tiles_plan_start(TilePlanJob& job);
   int tl_bw = -1;  // half bandwidth in the band order (reported), -1: no plan
   TileView tl_view;
   TileHost tl_host;
@@ -280,7 +278,7 @@ struct Domain {
   DVec<double> tl_A, tl_G, tl_Y, tl_X, tl_v;  // tiles, sweep vectors, 4 PCG vectors of a second right-hand side
   hipGraph_t tl_fg = nullptr, tl_sg[2] = {nullptr, nullptr};
   hipGraphExec_t tl_fe = nullptr, tl_se[2] = {nullptr, nullptr};
-  void tiles_setup(int bw);
+  void tiles_setup(TilePlanJob& job, int bw);
   bool cg_wide_on = true;
   // the current matrix's band factor (either kind) met a pivot that is not
   // positive (an indefinite tangent past a peak): its solves fall back to
