@@ -207,7 +207,11 @@ int  xg_spmv_config(xg_domain* d, int format, int lanes);
                           equations are preconditioned by their exact tiled
                           sparse factor in nested-dissection order (one or
                           two PCG iterations per solve) where it fits in
-                          2 x 4 GiB; a factor estimated above 3 ms is first
+                          2 x 4 GiB (XG_TILE_MIB in the environment: in so
+                          many MiB); without device memory for it the model
+                          goes on without it.  The memory is taken at xg_setup
+                          for a factor that the first solve uses, else by the
+                          first solve that does.  A factor estimated above 3 ms is first
                           formed when a solve without it has cost as much,
                           and used from then on until revertToStart; on by
                           default                                           */
@@ -275,9 +279,9 @@ int  xg_solve(xg_domain* d, const double* B, double* X);
    xg_solve; every PCG work buffer (staging of B and X, the six iteration
    vectors, the block-Jacobi inverses or the one-workgroup band factor,
    partial sums, scalars) comes from a fixed 128 MiB device array per GPU,
-   looked up at xg_create; the tiled factor (XG_CG_WIDE) uses the
-   domain's own buffers, allocated at xg_setup; the kernels are launched
-   one by one (no graph).  A system whose buffers do not fit (about 1.1 M
+   looked up at xg_create; the tiled factor (XG_CG_WIDE) is used where its
+   memory is already taken (by xg_setup or an earlier solve); the kernels are
+   launched one by one (no graph).  A system whose buffers do not fit (about 1.1 M
    equations with nodal 3x3 blocks) is XG_ERR_ARG.  Calls that overlap on
    one GPU share that array and race.                                       */
 int  xg_solve_noalloc(xg_domain* d, const double* B, double* X);

@@ -8,6 +8,7 @@ import time
 
 import numpy as np
 import pytest
+import torch
 
 from tests import _oracle
 from xara_amd import _lib, meshes
@@ -177,3 +178,81 @@ def test_failed_setup_leaves_no_thread():
         assert g.counters()["band_bw"] > 0
         g.close()
     assert np.array_equal(*X)
+
+
+def frame_model(size, integrator):
+    m = Model(3, 6)
+    fr = meshes.rc_frame_3d(*size)
+    meshes.build_rc_frame_3d(m, fr)
+    m.system("GpuBlockPCG", 1e-12, 20000)
+    if integrator == "Newmark":
+        m.masses(fr["load_tags"], np.tile([1.0, 1.0, 1.0, 0, 0, 0], (len(fr["load_tags"]), 1)))
+    m.integrator(integrator, *((0.5, 0.25) if integrator == "Newmark" else (1.0,)))
+    return m
+
+
+def taken(make):
+    """(model set up, device bytes its set-up took)"""
+    m = make()
+    free = torch.cuda.mem_get_info()[0]
+    m.setup()
+    return m, free - torch.cuda.mem_get_info()[0]
+
+
+def test_factor_memory_is_taken_when_a_solve_uses_it():
+    """A model set up as a transient takes no memory for the factor (2 x 57
+    MB for this 9 x 9 x 12 frame); its first static solve does, and is the one
+    of a model set up for static steps.  The allocation-free solve before it
+    goes without the factor."""
+    print("case: factor memory, 9 x 9 x 12 frame", flush=True)
+    frame_model((3, 3, 6), "LoadControl").setup()
+    st, a = taken(lambda: frame_model((9, 9, 12), "LoadControl"))
+    tr, b = taken(lambda: frame_model((9, 9, 12), "Newmark"))
+    assert a - b > 90 << 20
+    B = np.random.default_rng(0).normal(size=st.neq)
+    st.form_tangent(values=False)
+    X = st.solve(B)
+    tr.integrator("LoadControl", 1.0)
+    tr.form_tangent(values=False)
+    Xn = np.zeros_like(X)
+    assert tr._b.solve_noalloc(tr._h, B.ctypes.data_as(_lib.P_D), Xn.ctypes.data_as(_lib.P_D)) == 0
+    assert tr.counters()["band_bw"] == -1 and relerr(Xn, X) <= 1e-8
+    assert np.array_equal(tr.solve(B), X)
+    assert tr.counters()["band_bw"] == st.counters()["band_bw"] > 63
+    assert tr._b.solve_noalloc(tr._h, B.ctypes.data_as(_lib.P_D), Xn.ctypes.data_as(_lib.P_D)) == 0
+    assert np.array_equal(Xn, X)
+    st.close()
+    tr.close()
+
+
+@pytest.mark.parametrize("case", [("brick", 25), ("quad", 40, 7), ("frame", 5, 5, 8)],
+                         ids=lambda c: "_".join(map(str, c)))
+def test_without_memory_for_the_factor(case, monkeypatch):
+    """A model whose factor finds no memory (here: more than XG_TILE_MIB
+    allows) is set up and solved as without the factor: the band factor where
+    the band is narrow, else block Jacobi, step for step."""
+    print(f"case: no memory for the factor {case}", flush=True)
+    ndm, ndf = {"quad": (2, 2), "brick": (3, 3), "frame": (3, 6)}[case[0]]
+    runs = []
+    for mib in (None, "1"):
+        if mib:
+            monkeypatch.setenv("XG_TILE_MIB", mib)
+        m = Model(ndm, ndf)
+        node, dof, incr, _ = build(case, m)
+        m.system("GpuBlockPCG", 1e-12, 20000)
+        m.cg_config(wide=mib is not None)
+        if case[0] == "brick":
+            m.test("NormUnbalance", 1e-7, 30)
+            m.integrator("LoadControl", 93.0)
+        else:
+            if case[0] == "quad":
+                m.load(node, 0.0, 1.0)
+            m.test("NormUnbalance", 1e-6 if case[0] == "quad" else 1e-3, 30)
+            m.integrator("DisplacementControl", node, dof, incr)
+        m.setup()
+        assert m.analyze(3) == 0
+        c = m.counters()
+        runs.append((m.trial_disp(), c["cg_iters"], c["band_bw"]))
+        m.close()
+    assert np.array_equal(runs[0][0], runs[1][0]) and runs[0][1:] == runs[1][1:]
+    assert 0 < runs[1][2] <= 63 if case[0] == "quad" else runs[1][2] == -1

@@ -983,16 +983,18 @@ int Domain::solve_wide(int R, const double* const* b, double* const* x, const Cg
   return status;
 }
 
+bool Domain::tiles_plan(TilePlan& P) const {
+  const long long max_tiles = (long long)(kTileMaxBytes / (sizeof(double) * kTile * kTile));
+  return tile_plan(num.neq, num.rowptr, num.colind, nnode, ndf, ndm, num.eq, crd_h, max_tiles, 1e300, P);
+}
+
 // Starts the tiled factorisation's plan (host code) on a thread of its own:
 // it reads the numbering and the coordinates, which the rest of the set-up
-// leaves alone.  Without a thread to spare it runs in tiles_setup().
+// leaves alone.  Without a thread to spare it runs in tiles_take().
 void Domain::tiles_plan_start(TilePlanJob& job) {
-  const int n = num.neq;
-  if (n < kTileMinEqn || n > kTileMaxEqn) return;
-  auto build = [this, n, &job] {
-    const long long max_tiles = (long long)(kTileMaxBytes / (sizeof(double) * kTile * kTile));
-    return tile_plan(n, num.rowptr, num.colind, nnode, ndf, ndm, num.eq, crd_h, max_tiles, 1e300, job.plan);
-  };
+  tl_planned = false;
+  if (num.neq < kTileMinEqn || num.neq > kTileMaxEqn || integ == 3) return;
+  auto build = [this, &job] { return tiles_plan(job.plan); };
   try {
     job.done = std::async(std::launch::async, build);
   } catch (const std::system_error&) {
@@ -1000,16 +1002,45 @@ void Domain::tiles_plan_start(TilePlanJob& job) {
   }
 }
 
-// Takes the system into the tiled factorisation where its plan fits: the
-// device arrays of its launches.
-void Domain::tiles_setup(TilePlanJob& job, int bw) {
-  if (!job.done.valid() || !job.done.get()) return;
-  const TilePlan& P = job.plan;
-  const int n = num.neq;
+// The plan, where it fits, kept until tiles_alloc() (and what the choice of
+// path needs of it); a plan that found no host memory is none.
+void Domain::tiles_take(TilePlanJob& job) {
+  tl_planned = true;
+  bool ok = false;
+  try {
+    ok = job.done.get();
+  } catch (const std::bad_alloc&) {
+  }
+  if (!ok) return;
+  tl_plan = std::make_shared<TilePlan>(std::move(job.plan));
+  const TilePlan& P = *tl_plan;
   tl_factor_us = 25.0 * P.nlev + P.flops / 30e6;
   tl_iter_us = 15.0 + 0.55 * 8.0 * (double)num.colind.size() / 3.4e6;
   tl_cap = std::max(cg_chunk, (int)(tl_factor_us / tl_iter_us));
   tl_on = false;
+  tl_bw = order_bw;
+}
+
+// Before a solve that may allocate: the plan of a model set up for a
+// transient, and the factor's memory, when this solve would take the factor.
+void Domain::tiles_ready() {
+  if (!cg_small_on || !cg_wide_on || integ == 3 || tl_mem) return;
+  if (!tl_planned) {
+    tl_planned = true;
+    if (num.neq >= kTileMinEqn && num.neq <= kTileMaxEqn) {
+      TilePlanJob job;
+      job.done = std::async(std::launch::deferred, [&] { return tiles_plan(job.plan); });
+      tiles_take(job);
+    }
+  }
+  if (tl_usable() && (!tl_big() || tl_on)) tiles_alloc();
+}
+
+// The device arrays of the factor and its launches.  Where the device has no
+// memory for them the model goes on without the factor.
+void Domain::tiles_alloc() {
+  const TilePlan& P = *tl_plan;
+  const int n = num.neq;
   // panel tasks: a workgroup per row tile, several where a level has many
   // (every workgroup of a column inverts its diagonal block itself)
   std::vector<int4> task;
@@ -1044,6 +1075,17 @@ void Domain::tiles_setup(TilePlanJob& job, int bw) {
       {&tl_view.fwsrc, &P.fwsrc}, {&tl_view.fwg, &P.fwg},     {&tl_view.fwk, &P.fwk},     {&tl_view.bwcol, &P.bwcol},
       {&tl_view.bwsrc, &P.bwsrc}, {&tl_view.bwg, &P.bwg},     {&tl_view.bwr, &P.bwr}};
   for (auto& q : parts) all.insert(all.end(), q.second->begin(), q.second->end());
+  const size_t doubles = (size_t)P.tiles() * kTile * kTile, np = (size_t)kTile * P.nt;
+  // XG_TILE_MIB in the environment bounds what A and G may take together
+  const char* env = std::getenv("XG_TILE_MIB");
+  const bool allowed = !env || (double)(2 * doubles * sizeof(double)) <= std::atof(env) * 1048576.0;
+  if (!allowed || !tl_A.try_resize(doubles) || !tl_G.try_resize(doubles) || !tl_Y.try_resize(2 * np) ||
+      !tl_X.try_resize(2 * np) || !tl_v.try_resize(4 * (size_t)n) || !tl_ints.try_resize(all.size()) ||
+      !tl_task.try_resize(task.size())) {
+    tiles_release();
+    return;
+  }
+  pc_buffers();
   tl_ints.upload(all, stream);
   tl_task.upload(task, stream);
   XG_HIP(hipStreamSynchronize(stream));
@@ -1054,13 +1096,19 @@ void Domain::tiles_setup(TilePlanJob& job, int bw) {
   }
   tl_view.task = tl_task.p;
   tl_view.nt = P.nt;
-  const size_t doubles = (size_t)P.tiles() * kTile * kTile, np = (size_t)kTile * P.nt;
-  tl_A.resize(doubles);
-  tl_G.resize(doubles);
-  tl_Y.resize(2 * np);
-  tl_X.resize(2 * np);
-  tl_v.resize(4 * (size_t)n);
-  tl_bw = bw;
+  tl_plan.reset();
+  tl_mem = true;
+}
+
+void Domain::tiles_release() {
+  for (auto* v : {&tl_A, &tl_G, &tl_Y, &tl_X, &tl_v}) v->release();
+  tl_ints.release();
+  tl_task.release();
+  tl_view = TileView{};
+  tl_plan.reset();
+  tl_mem = tl_on = false;
+  tl_factor_us = 0;
+  tl_bw = -1;
 }
 
 // Half bandwidth of the pattern under an equation order (pinv: position of
@@ -1075,8 +1123,7 @@ static int band_width(const Numbering& num, const std::vector<int>& pinv) {
 
 void Domain::band_order(TilePlanJob& plan) {
   band_bw = -1;
-  tl_bw = -1;
-  tl_factor_us = 0;
+  tiles_release();
   pc_cache = pc_fresh = false;
   pc_vals.release();
   band_pinv.release();
@@ -1084,10 +1131,6 @@ void Domain::band_order(TilePlanJob& plan) {
   band2.release();
   band_L.release();
   band_Lr.release();
-  for (auto* v : {&tl_A, &tl_G, &tl_Y, &tl_X, &tl_v}) v->release();
-  tl_ints.release();
-  tl_task.release();
-  tl_view = TileView{};
   const int n = num.neq;
   if (n == 0 || n > kTileMaxEqn) return;
   std::vector<int> ident(n);
@@ -1127,8 +1170,9 @@ void Domain::band_order(TilePlanJob& plan) {
       pinv = geo;
     }
   }
-  tiles_setup(plan, best);
-  if (tl_bw >= 0) pc_buffers();
+  order_bw = best;
+  if (plan.done.valid()) tiles_take(plan);
+  tiles_ready();
   if (best > 63 || n > kBandMaxEqn) return;
   band_bw = best;
   band_pinv.upload(pinv, stream);
@@ -1146,7 +1190,8 @@ void Domain::pc_buffers() {
   const char* env = std::getenv("XG_PC_REUSE");
   pc_reuse_on = !(env && env[0] == '0');
   if (!pc_reuse_on) return;
-  pc_vals.resize(std::max<size_t>(num.colind.size(), 1));
+  // (without memory for it every matrix is factored)
+  (void)pc_vals.try_resize(std::max<size_t>(num.colind.size(), 1));
 }
 
 // Destroys the captured chunks once the stream has drained: a replay still
@@ -1210,6 +1255,7 @@ void Domain::cg_chunk_run(int iters, int it0, int L, int bw, double* x, const Cg
 // results); otherwise one after the other.
 int Domain::solve_pair(const double* b1, double* x1, const double* b2, double* x2) {
   const int n = num.neq;
+  tiles_ready();
   if (n > 0 && wide_active()) {
     const CgBufs w = cg_bufs();
     precond_setup(w);
@@ -1284,6 +1330,8 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
   const int n = num.neq;
   if (n == 0) return 0;
   const int bw = (system == XG_SYSTEM_PCG_BLOCKJACOBI) ? ndf : 1;
+  const bool own = w.pcbad == pcbad;  // not the allocation-free solve
+  if (own) tiles_ready();
   precond_setup(w);
   int conv = 0, it = 0, brk = 0;
   double rr = 0, bb = 0;
@@ -1323,7 +1371,7 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
     cg_start(stream, n, bs, xs, w.r0, w.z, w.p, bw, sweep ? w.binvs : w.binv, bfirst.p, bsize.p, w.part,
              rtol * rtol, maxit, w.scal, warm ? w.q : nullptr);
     int issued = 0, next = cg_chunk;
-    const int cap = tl_usable() && tl_big() && !tl_on ? tl_cap : INT_MAX;
+    int cap = tl_usable() && tl_big() && !tl_on && (own || tl_mem) ? tl_cap : INT_MAX;
     const int L = lanes();
     while (true) {
       read_status(w);
@@ -1337,9 +1385,13 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
       if (issued >= maxit + 1) break;
       if (issued >= cap) {
         // worth a factor: this solve again, and the later ones, with it
-        counters.cg_iters += it;
         tl_on = true;
-        return solve_with(b, x, w, graphs);
+        if (own) tiles_ready();
+        if (wide_active()) {
+          counters.cg_iters += it;
+          return solve_with(b, x, w, graphs);
+        }
+        cap = INT_MAX;  // there is no memory for it
       }
       // chunks double (up to 8x cg_chunk) while the solve goes on: fewer
       // host round trips on long solves; iterations issued past
@@ -1527,6 +1579,7 @@ int Domain::newton() {
   bool first = true;
   do {
     form_tangent();
+    tiles_ready();
     if (integ == 2 && (band_active() || wide_active())) {
       // DisplacementControl::update solves for the reference load with the
       // same matrix: both solves at once

@@ -79,6 +79,8 @@ struct FiberSecDef {
   bool centroid = true;
 };
 
+struct TilePlan;
+
 struct Domain {
   int ndm = 0, ndf = 0, device = 0;
   hipStream_t stream = nullptr;
@@ -246,7 +248,7 @@ struct Domain {
   struct TilePlanJob;  // the tiled factor's plan, built on a thread beside the rest of the set-up
   void band_order(TilePlanJob& plan);
   // tiled sparse factorisation (xg_tiles.hip), the exact preconditioner
-  // under the static integrators of the systems tiles_setup() takes (a
+  // under the static integrators of the systems tiles_take() accepts (a
   // transient's K + c3 M is well conditioned by the mass term: block Jacobi
   // converges in tens of iterations there).  A solve takes one or two PCG
   // iterations (solve_wide); factor and sweeps are replayed from captured
@@ -269,8 +271,21 @@ struct Domain {
   int tl_cap = 0;
   bool tl_big() const { return tl_factor_us > kTileBigUs; }
   bool tl_usable() const { return cg_small_on && cg_wide_on && !wb_failed && tl_bw >= 0 && integ != 3; }
+  bool tiles_plan(TilePlan& P) const;
   void tiles_plan_start(TilePlanJob& job);
-  int tl_bw = -1;  // half bandwidth in the band order (reported), -1: no plan
+  void tiles_take(TilePlanJob& job);
+  // The plan is made at set-up (for a model set up as a transient, at its
+  // first static solve).  The memory, up to 2 x 4 GiB, is taken at set-up
+  // only for a factor that the first solve uses; else by the first solve
+  // that does, so that state determination, transients and solids that stay
+  // with block Jacobi do without.  The allocation-free solve never takes it.
+  void tiles_ready();
+  void tiles_alloc();
+  void tiles_release();
+  std::shared_ptr<TilePlan> tl_plan;  // until its arrays are on the device
+  bool tl_planned = false, tl_mem = false;
+  int order_bw = 0;  // half bandwidth in the band order
+  int tl_bw = -1;  // half bandwidth in the band order (reported), -1: no factor
   TileView tl_view;
   TileHost tl_host;
   DVec<int> tl_ints;
@@ -278,7 +293,6 @@ struct Domain {
   DVec<double> tl_A, tl_G, tl_Y, tl_X, tl_v;  // tiles, sweep vectors, 4 PCG vectors of a second right-hand side
   hipGraph_t tl_fg = nullptr, tl_sg[2] = {nullptr, nullptr};
   hipGraphExec_t tl_fe = nullptr, tl_se[2] = {nullptr, nullptr};
-  void tiles_setup(TilePlanJob& job, int bw);
   bool cg_wide_on = true;
   // the current matrix's band factor (either kind) met a pivot that is not
   // positive (an indefinite tangent past a peak): its solves fall back to
@@ -294,7 +308,7 @@ struct Domain {
   const void* pc_cache_key = nullptr;
   const void* pc_fresh_key = nullptr;
   long long pc_reuses = 0;
-  bool wide_active() const { return tl_usable() && (!tl_big() || tl_on); }
+  bool wide_active() const { return tl_usable() && (!tl_big() || tl_on) && tl_mem; }
   void tiles_form(int* bad);
   void pc_buffers();
   void tiles_apply(int k, const double* const* r, double* const* z, bool graphs);

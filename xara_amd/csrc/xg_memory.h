@@ -25,6 +25,22 @@ struct DVec {
     n = count;
     if (count) XG_HIP(hipMalloc((void**)&p, count * sizeof(T)));
   }
+  // false, holding nothing, where the device has no memory for it
+  bool try_resize(size_t count) {
+    if (count == n && (p || !count)) return true;
+    release();
+    if (count) {
+      const hipError_t e = hipMalloc((void**)&p, count * sizeof(T));
+      if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();  // handled here: not the next caller's error
+        p = nullptr;
+        return false;
+      }
+      XG_HIP(e);
+    }
+    n = count;
+    return true;
+  }
   void zero(hipStream_t s) {
     if (n) XG_HIP(hipMemsetAsync(p, 0, n * sizeof(T), s));
   }
