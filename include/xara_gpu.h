@@ -79,8 +79,9 @@ typedef struct xg_counters {
                                  order when an exact factor (band or tiled)
                                  preconditions the PCG, -1 otherwise       */
   long long band_fallbacks;   /* matrices whose exact factor met a pivot
-                                 that is not positive and were solved with
-                                 block Jacobi instead                      */
+                                 that is not positive, or with which the
+                                 PCG failed, solved with block Jacobi
+                                 instead                                   */
   long long band_reuses;      /* assembled matrices equal bit for bit to the
                                  last one factored, whose factor was
                                  kept instead of formed again              */

@@ -928,7 +928,11 @@ void Domain::tiles_apply(int k, const double* const* r, double* const* z, bool g
 // |r| <= rtol |b| like the other paths.  The factor makes the first iterate
 // the direct solution up to rounding, so a solve takes one or two
 // iterations.  The scalars stay on the device; the host reads them once per
-// iteration.
+// iteration.  A factor whose pivots are all positive can still be far from
+// the matrix's inverse, where the smallest of them are rounding (a model
+// without enough supports under loads in balance, which block Jacobi
+// solves): a solve that breaks down, or has not converged after
+// kTileMaxIters, drops it.
 int Domain::solve_wide(int R, const double* const* b, double* const* x, const CgBufs& w, bool graphs,
                        unsigned warm) {
   const int n = num.neq;
@@ -953,7 +957,7 @@ int Domain::solve_wide(int R, const double* const* b, double* const* x, const Cg
   }
   tiles_pcg_start(stream, n, R, P, tol2);
   int bad = warm ? read() : 0;  // a guess within the tolerance ends its solve before the first iteration
-  for (int it = 0; it < maxit && !bad; it++) {
+  for (int it = 0; it < std::min(maxit, kTileMaxIters) && !bad; it++) {
     const double* rs[2];
     double* zs[2];
     int k = 0;
@@ -972,15 +976,17 @@ int Domain::solve_wide(int R, const double* const* b, double* const* x, const Cg
   }
   if (!settled) bad = read();
   if (bad) return bad;
-  int status = 0;
+  bool ok = true;
   for (int s = 0; s < R; s++) {
-    const TileScal& S = T[s];
-    counters.solves++;
-    counters.cg_iters += S.iters;
-    counters.last_cg_relres = S.bb > 0 ? std::sqrt(S.rr / S.bb) : 0.0;
-    if (S.fail || (S.bb > 0 && !(S.rr <= tol2 * S.bb))) status = XG_BAD_LINEAR_SOLVE;
+    counters.cg_iters += T[s].iters;
+    ok = ok && !T[s].fail && (!(T[s].bb > 0) || T[s].rr <= tol2 * T[s].bb);
   }
-  return status;
+  if (!ok) return drop_factor();
+  for (int s = 0; s < R; s++) {
+    counters.solves++;
+    counters.last_cg_relres = T[s].bb > 0 ? std::sqrt(T[s].rr / T[s].bb) : 0.0;
+  }
+  return 0;
 }
 
 bool Domain::tiles_plan(TilePlan& P) const {
@@ -1319,10 +1325,15 @@ int Domain::precond_settle(const CgBufs& w) {
     }
     return 0;
   }
-  if (!band_active() && !wide_active()) return -1;
+  return band_active() || wide_active() ? drop_factor() : -1;
+}
+
+// The exact factor of the current matrix gives way to the PCG without it.
+int Domain::drop_factor() {
   wb_failed = true;
   wb_fallbacks++;
   pc_done = nullptr;
+  pc_cache = false;
   return 1;
 }
 

@@ -294,9 +294,10 @@ struct Domain {
   hipGraph_t tl_fg = nullptr, tl_sg[2] = {nullptr, nullptr};
   hipGraphExec_t tl_fe = nullptr, tl_se[2] = {nullptr, nullptr};
   bool cg_wide_on = true;
-  // the current matrix's band factor (either kind) met a pivot that is not
-  // positive (an indefinite tangent past a peak): its solves fall back to
-  // the PCG without it until the next assembly
+  // the current matrix's exact factor (band or tiled) met a pivot that is not
+  // positive (an indefinite tangent past a peak), or the PCG failed with the
+  // tiled one: its solves fall back to the PCG without it until the next
+  // assembly
   bool wb_failed = false;
   long long wb_fallbacks = 0;
   // the values of the matrix whose band factor (either kind) the domain's
@@ -313,7 +314,8 @@ struct Domain {
   void pc_buffers();
   void tiles_apply(int k, const double* const* r, double* const* z, bool graphs);
   // warm: bit s set when x[s] holds a guess to start right-hand side s from
-  // 1: the factor met a bad pivot (precond_settle)
+  // 1: the factor met a bad pivot, or the PCG failed with it, and is dropped
+  static constexpr int kTileMaxIters = 32;
   int solve_wide(int R, const double* const* b, double* const* x, const CgBufs& w, bool graphs, unsigned warm = 0);
   // the preconditioner's buffers last formed from the current matrix
   // (nullptr: the matrix changed since), so repeated solves of one matrix
@@ -329,6 +331,7 @@ struct Domain {
   // after read_status: 0 the preconditioner is good, 1 an exact factor met a
   // bad pivot and is dropped (solve again without it), -1 no preconditioner
   int precond_settle(const CgBufs& w);
+  int drop_factor();
   void incr_disp(const double* dU_dev, double scale = 1.0);
   void commit();  // queued, like every operation the analysis loop issues
   void revert();
