@@ -283,3 +283,44 @@ def test_factor_without_enough_supports_gives_way(size):
             b = m.spmv(1e-3 * rng.normal(size=m.neq))
             assert np.linalg.norm(m.spmv(m.solve(b)) - b) <= 1.1e-10 * np.linalg.norm(b)
             m.close()
+
+
+@pytest.mark.parametrize("wide", [True, False], ids=["tiled", "band"])
+@pytest.mark.parametrize("control", ["load", "displacement"])
+def test_dropped_factor_keeps_the_warm_start(control, wide):
+    """Elastic fibers of a negative modulus: no pivot is positive, so the
+    exact factor is dropped for every matrix, and block Jacobi solves the
+    negative definite system.  A step's first solve (LoadControl) and the
+    solves for the reference load (DisplacementControl; with the band factor
+    the predictor's only) still start from the last one's solution: of 4
+    solves 3 end at once, of 12 solves 7 (3)."""
+    print(f"case: warm start without the factor, {control} {wide}", flush=True)
+    fr = meshes.rc_frame_2d(24, 15)
+    its = []
+    for warm in (True, False):
+        m = Model(2, 3)
+        m.nodes(fr["node_tags"], fr["crds"])
+        m.fix_many(fr["fixed_nodes"], np.ones((len(fr["fixed_nodes"]), 3), np.int32))
+        m.uniaxialMaterial("Elastic", 1, -2e5)
+        m.section("Fiber", 1, [(y, 0.0, 1e4, 1) for y in (-200.0, -100.0, 100.0, 200.0)])
+        m.geomTransf("Linear", 1)
+        conn = np.concatenate([fr["columns"], fr["beams"]])
+        m.elements("dispBeamColumn", np.arange(1, len(conn) + 1), conn, 1, 1, 5)
+        P = np.zeros((len(fr["floor_nodes"]), 3))
+        P[:, 0] = 1.0
+        m.loads(fr["floor_nodes"], P)
+        m.system("GpuBlockPCG", 1e-8, 50000)
+        m.cg_config(warm=warm, wide=wide)
+        m.test("NormUnbalance", 1e-2, 20)
+        if control == "load":
+            m.integrator("LoadControl", 10.0)
+        else:
+            m.integrator("DisplacementControl", fr["roof"], 1, 5.0)
+        m.setup()
+        assert m.neq > 1024 and 0 < m.counters()["band_bw"] <= 63
+        assert m.analyze(4) == 0
+        c = m.counters()
+        assert c["band_fallbacks"] > 0
+        its.append(c["cg_iters"])
+        m.close()
+    assert its[0] < (0.6 if wide or control == "load" else 0.8) * its[1]

@@ -981,7 +981,10 @@ int Domain::solve_wide(int R, const double* const* b, double* const* x, const Cg
     counters.cg_iters += T[s].iters;
     ok = ok && !T[s].fail && (!(T[s].bb > 0) || T[s].rr <= tol2 * T[s].bb);
   }
-  if (!ok) return drop_factor();
+  if (!ok) {
+    (void)drop_factor();
+    return 2;
+  }
   for (int s = 0; s < R; s++) {
     counters.solves++;
     counters.last_cg_relres = T[s].bb > 0 ? std::sqrt(T[s].rr / T[s].bb) : 0.0;
@@ -1261,6 +1264,7 @@ void Domain::cg_chunk_run(int iters, int it0, int L, int bw, double* x, const Cg
 // results); otherwise one after the other.
 int Domain::solve_pair(const double* b1, double* x1, const double* b2, double* x2) {
   const int n = num.neq;
+  bool warm2 = false;
   tiles_ready();
   if (n > 0 && wide_active()) {
     const CgBufs w = cg_bufs();
@@ -1269,8 +1273,10 @@ int Domain::solve_pair(const double* b1, double* x1, const double* b2, double* x
     double* xs[2] = {x1, x2};
     // the second right-hand side is DisplacementControl's reference load:
     // its last solution in x2 is the start
-    const int r = solve_wide(2, bs, xs, w, cg_graph_on, (cg_warm_on && dc_hat_valid) ? 2u : 0u);
+    warm2 = cg_warm_on && dc_hat_valid;
+    const int r = solve_wide(2, bs, xs, w, cg_graph_on, warm2 ? 2u : 0u);
     if (r <= 0) return r;
+    warm2 = warm2 && r == 1;
   } else if (n > 0 && band_active() && band2.n >= (size_t)5 * n) {
     const CgBufs w = cg_bufs();
     precond_setup(w);
@@ -1297,9 +1303,9 @@ int Domain::solve_pair(const double* b1, double* x1, const double* b2, double* x
     }
   }
   // no exact factor, or one that gave way to the PCG without it: one solve
-  // after the other
+  // after the other, the second from its guess where that is still there
   const int r = solve(b1, x1);
-  return r < 0 ? r : solve(b2, x2);
+  return r < 0 ? r : solve_from(b2, x2, warm2);
 }
 
 // The status block to its pinned copy (and a workspace's own flag and
@@ -1358,7 +1364,7 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
     const double* bs[1] = {b};
     double* xs[1] = {x};
     const int r = solve_wide(1, bs, xs, w, graphs, warm ? 1u : 0u);
-    return r > 0 ? solve_with(b, x, w, graphs) : r;
+    return r > 0 ? solve_with(b, x, w, graphs, warm && r == 1) : r;
   } else if (small_path()) {
     // the whole solve in one workgroup, one launch
     cg_solve_small(stream, n, (long long)num.colind.size(), rowptr.p, colind.p, vals.p, b, x, bw, w.binv, bfirst.p,
@@ -1418,7 +1424,7 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
     }
   }
   if (bad < 0) return XG_BAD_LINEAR_SOLVE;
-  if (bad > 0) return solve_with(b, x, w, graphs);  // without the factor, from zero
+  if (bad > 0) return solve_with(b, x, w, graphs, warm);  // without the band factor: x is as it was
   cg_parse_scal(stat_h + kStCg, &conv, &it, &rr, &bb, &brk);
   counters.solves++;
   counters.cg_iters += it;

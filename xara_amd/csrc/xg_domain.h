@@ -314,7 +314,8 @@ struct Domain {
   void pc_buffers();
   void tiles_apply(int k, const double* const* r, double* const* z, bool graphs);
   // warm: bit s set when x[s] holds a guess to start right-hand side s from
-  // 1: the factor met a bad pivot, or the PCG failed with it, and is dropped
+  // 1: the factor met a bad pivot and is dropped (a guess in x is still
+  // there), 2: the PCG failed with it, and it is dropped
   static constexpr int kTileMaxIters = 32;
   int solve_wide(int R, const double* const* b, double* const* x, const CgBufs& w, bool graphs, unsigned warm = 0);
   // the preconditioner's buffers last formed from the current matrix
