@@ -19,6 +19,11 @@ FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950",
     # keep the compiler from forming packed-FP32 instructions
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # loops of the host code begin on 32 bytes: the index maps of the set-up are
+    # short loops over millions of entries, and unaligned they ran by turns 10%
+    # slower (24^3 bricks, whole preparation 197 or 220 ms) as code before them
+    # grew or shrank
+    "-Xarch_host", "-falign-loops=32",
     # matrix instructions accumulate in the ordinary registers (they are moved
     # and selected between products in the tiled factorisation)
     "-mllvm", "-amdgpu-mfma-vgpr-form",
