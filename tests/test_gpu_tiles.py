@@ -324,3 +324,45 @@ def test_dropped_factor_keeps_the_warm_start(control, wide):
         its.append(c["cg_iters"])
         m.close()
     assert its[0] < (0.6 if wide or control == "load" else 0.8) * its[1]
+
+
+def test_large_solid_tries_block_jacobi_again(monkeypatch):
+    """A solid that has gone on with the factor returns to block Jacobi after
+    16 factored matrices: elastic unloading after plastic steps takes 16
+    factors and then iterations; while the steps stay hard every solve is
+    finished by the factor."""
+    print("case: large solid 25^3 unloaded", flush=True)
+    monkeypatch.setenv("XG_PC_REUSE", "0")  # count a factor for every matrix
+    m = Model(3, 3)
+    mesh = meshes.brick_cube(25)
+    meshes.build_brick_cube(m, mesh)
+    m.system("GpuBlockPCG", 1e-10, 20000)
+    m.test("NormUnbalance", 1e-7, 30)
+    m.integrator("LoadControl", 93.0)
+    m.setup()
+    b = np.zeros(m.neq)
+    m.set_load_factor(1.0)
+    b[:] = m.form_unbalance()
+    m.set_load_factor(0.0)
+    assert m.analyze(3) == 0
+    U = m.trial_disp()
+
+    def solves(scale, n):
+        its, on = [], []
+        m.set_trial_disp(scale * U)
+        m.update()
+        for _ in range(n):
+            m.form_tangent(values=False)
+            c = m.counters()["cg_iters"]
+            X = m.solve(b)
+            its.append(m.counters()["cg_iters"] - c)
+            on.append(m.counters()["band_bw"] > 0)
+        return its, on, X
+    its, on, X = solves(1.02, 40)  # loading on: block Jacobi alone would not do
+    assert on == [True] * 40
+    assert 1 <= sum(i > 30 for i in its) <= 3  # the tries
+    its, on, Xe = solves(0.98, 20)
+    assert max(its[:1]) <= 3 and on[0] and not on[-1]
+    assert on == sorted(on, reverse=True) and 1 <= sum(on) <= 16
+    assert min(its[sum(on):]) > 30
+    m.close()

@@ -836,6 +836,7 @@ void Domain::form_tangent() {
   sym_stale = true;
   pc_done = nullptr;
   wb_failed = false;
+  if (tl_formed >= kTileRetry) tl_on = false;
   // Newmark::formNodTangent: c2 C + c3 M of the nodal masses (C = alphaM M)
   if (integ == 3) launch_add_diag(stream, nmass_eq, mass_pos.p, mass_val.p, nm_c3 + nm_c2 * alphaM, vals.p);
 }
@@ -880,6 +881,7 @@ void Domain::precond_setup(const CgBufs& w) {
   }
   if (wide) {
     tiles_form(w.pcbad);
+    tl_formed++;
   } else if (band) {
     band_factor(stream, num.neq, band_bw, rowptr.p, colind.p, vals.p, band_pinv.p, w.bandA, w.bandL, w.bandLr,
                 w.pcbad);
@@ -1023,9 +1025,8 @@ void Domain::tiles_take(TilePlanJob& job) {
   if (!ok) return;
   tl_plan = std::make_shared<TilePlan>(std::move(job.plan));
   const TilePlan& P = *tl_plan;
-  tl_factor_us = 25.0 * P.nlev + P.flops / 30e6;
-  tl_iter_us = 15.0 + 0.55 * 8.0 * (double)num.colind.size() / 3.4e6;
-  tl_cap = std::max(cg_chunk, (int)(tl_factor_us / tl_iter_us));
+  tl_factor_us = 31.0 * P.nlev + P.flops / 48e6;
+  tl_iter_us = 12.0 + 1.8e-6 * (double)num.colind.size();
   tl_on = false;
   tl_bw = order_bw;
 }
@@ -1388,7 +1389,10 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
     cg_start(stream, n, bs, xs, w.r0, w.z, w.p, bw, sweep ? w.binvs : w.binv, bfirst.p, bsize.p, w.part,
              rtol * rtol, maxit, w.scal, warm ? w.q : nullptr);
     int issued = 0, next = cg_chunk;
-    int cap = tl_usable() && tl_big() && !tl_on && (own || tl_mem) ? tl_cap : INT_MAX;
+    // whole chunks worth a factor
+    int cap = INT_MAX;
+    if (tl_usable() && tl_big() && !tl_on && (own || tl_mem))
+      cap = ((int)(tl_factor_us / tl_iter_us) / cg_chunk + 1) * cg_chunk;
     const int L = lanes();
     while (true) {
       read_status(w);
@@ -1403,6 +1407,7 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
       if (issued >= cap) {
         // worth a factor: this solve again, and the later ones, with it
         tl_on = true;
+        tl_formed = 0;
         if (own) tiles_ready();
         if (wide_active()) {
           counters.cg_iters += it;
@@ -1413,7 +1418,7 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
       // chunks double (up to 8x cg_chunk) while the solve goes on: fewer
       // host round trips on long solves; iterations issued past
       // convergence return at once
-      const int chunk = std::min(next, maxit + 1 - issued);
+      const int chunk = std::min({next, maxit + 1 - issued, cap - issued});
       cg_chunk_run(chunk, issued, L, bw, xs, w, graphs);
       issued += chunk;
       next = std::min(2 * next, 8 * cg_chunk);

@@ -253,22 +253,36 @@ struct Domain {
   // converges in tens of iterations there).  A solve takes one or two PCG
   // iterations (solve_wide); factor and sweeps are replayed from captured
   // graphs when cg_graph_on.
+  // Fewer equations: the one-workgroup band factor (k_band_factor_w), or
+  // block Jacobi (k_pcg_small) for bands above 63.  A new matrix and one solve,
+  // tiled / without, us: quad strips 120 equations 111 / 98, 256 133 / 149, 360
+  // 156 / 196, 528 175 / 266, 780 (bw 51) 185 / 1,756; 2D frames 180 129 / 115,
+  // 336 154 / 165, 540 159 / 241, 1,080 245 / 419; 3D frames 108 111 / 102, 216
+  // (bw 59) 142 / 517, 360 (bw 77) 183 / 1,016, 576 233 / 1,190; solids 300
+  // 151 / 347, 540 207 / 1,024.  From 385 on the tiled factor is the faster one
+  // for every band; bands up to 44 cross at about 300 equations, and wider ones
+  // would gain below 385 too.
   static constexpr int kTileMinEqn = 385, kTileMaxEqn = 1 << 18;
   static constexpr int kTilePanelGroups = 512;
   static constexpr size_t kTileMaxBytes = size_t(4) << 30;  // each of A and G
-  // A large solid's factor takes as long as hundreds of PCG iterations
-  // (tl_factor_us, tl_iter_us: fits to solids of 12^3 to 33^3 elements, 25 us
-  // per level and 30 TFLOP/s; 15 us per iteration and 3.4 TB/s of the
-  // product).  Above kTileBigUs such a model starts with block Jacobi, and a
-  // solve that has not converged after as many iterations as a factor is
-  // worth (tl_cap) goes on with the factor, as do the later ones until
-  // revertToStart: at most twice the better of the two on any solve, and
-  // mildly plastic steps (100 to 300 iterations at 28 us on 33^3) keep the
-  // cheap iterations where the factor takes 16 ms.
-  static constexpr double kTileBigUs = 3000.0;
+  // A large solid's factor takes as long as hundreds of PCG iterations: about
+  // tl_factor_us against tl_iter_us (31 us per level and 48 TFLOP/s; 12 us and
+  // 1.8 us per million entries).  Solids of 16^3 / 20^3 / 24^3 / 28^3 / 33^3 /
+  // 36^3 / 40^3: 1.16 / 2.14 / 3.75 / 6.40 / 12.2 / 18.4 / 30.2 ms, measured
+  // 1.05 / 2.17 / 3.93 / 6.64 / 12.6 / 18.6 / 30.3; an iteration from 24^3 on
+  // 18.0 / 21.6 / 27.7 / 32.4 / 40.0 us, measured 17.2 / 23.3 / 28.5 / 33.0 /
+  // 39.9.  Above kTileBigUs such a model starts with block Jacobi, and a solve
+  // that has not converged after as many iterations as a factor is worth goes
+  // on with the factor: at most about twice the better of the two for that
+  // solve.  The later solves keep the factor until revertToStart, or until
+  // kTileRetry matrices were factored: then block Jacobi is tried again (steps
+  // may have turned mild, 100 to 300 iterations), which costs a sixteenth
+  // where they have not.
+  static constexpr double kTileBigUs = 2800.0;
+  static constexpr int kTileRetry = 16;
   double tl_factor_us = 0, tl_iter_us = 1;
   bool tl_on = false;  // a solve has gone on with the factor
-  int tl_cap = 0;
+  int tl_formed = 0;   // matrices factored since
   bool tl_big() const { return tl_factor_us > kTileBigUs; }
   bool tl_usable() const { return cg_small_on && cg_wide_on && !wb_failed && tl_bw >= 0 && integ != 3; }
   bool tiles_plan(TilePlan& P) const;
