@@ -1542,10 +1542,10 @@ int Domain::new_step() {
   if (dc_incr < dc_min) dc_incr = dc_min;
   else if (dc_incr > dc_max) dc_incr = dc_max;
   form_tangent();
-  pick_on = true;
-  const int solved = solve_from(phat.p, dUhat.p, cg_warm_on && dc_hat_valid);
-  pick_on = false;
-  if (solved < 0) return XG_BAD_STEP;
+  {
+    const Pick pick(*this);
+    if (solve_from(phat.p, dUhat.p, cg_warm_on && dc_hat_valid) < 0) return XG_BAD_STEP;
+  }
   dc_hat_valid = true;
   const double dUahat = ((const double*)(stat_h + kStCtrl))[1];
   if (dUahat == 0.0) return XG_BAD_STEP;
@@ -1574,10 +1574,8 @@ int Domain::integ_update(const double* x) {
   const bool hat_ready = dc_hat_ready;
   dc_hat_ready = false;
   if (!hat_ready) {
-    pick_on = true;
-    const int solved = solve_from(phat.p, dUhat.p, cg_warm_on && dc_hat_valid);
-    pick_on = false;
-    if (solved < 0) return XG_BAD_STEP;
+    const Pick pick(*this);
+    if (solve_from(phat.p, dUhat.p, cg_warm_on && dc_hat_valid) < 0) return XG_BAD_STEP;
   }
   dc_hat_valid = true;
   // the last read_status brought both at the control DOF
@@ -1605,10 +1603,8 @@ int Domain::newton() {
     if (integ == 2 && (band_active() || wide_active())) {
       // DisplacementControl::update solves for the reference load with the
       // same matrix: both solves at once
-      pick_on = true;
-      const int solved = solve_pair(B.p, X.p, phat.p, dUhat.p);
-      pick_on = false;
-      if (solved < 0) return XG_BAD_LINEAR_SOLVE;
+      const Pick pick(*this);
+      if (solve_pair(B.p, X.p, phat.p, dUhat.p) < 0) return XG_BAD_LINEAR_SOLVE;
       dc_hat_ready = true;
     } else {
       // under LoadControl the first iteration of a step solves for the same

@@ -151,7 +151,14 @@ struct Domain {
   TileScal* tl_scal = nullptr;
   char *scal = nullptr, *scal2 = nullptr;  // CGScal of a solve, and of a second one beside it
   TileScal* tl_read() { return reinterpret_cast<TileScal*>(stat_h + kStTile); }
-  bool pick_on = false;  // read_status also brings ctrl
+  // while one lives, read_status also brings ctrl (a solve that throws must
+  // not leave that on: the next model's vectors may be shorter)
+  bool pick_on = false;
+  struct Pick {
+    Domain& d;
+    explicit Pick(Domain& dom) : d(dom) { d.pick_on = true; }
+    ~Pick() { d.pick_on = false; }
+  };
   int nblk = 0;
   // analysis configuration
   int system = XG_SYSTEM_PCG_JACOBI, numberer = XG_NUMBERER_RCM;
