@@ -1,12 +1,12 @@
-"""GPU parity of the wide-band Cholesky preconditioner (xg_wband.hip: the
-band of a system of more than 1,024 equations factored in 64 x 64 tiles,
-the PCG preconditioned by the exact factor) against the CPU oracle's direct
-solve: single solves on a 3D RC frame (half bandwidth above 63, several
-tiles per column) and on a quad strip of more than 16,384 equations (one
-tile below the diagonal), a DisplacementControl pushover whose two solves
-per Newton iteration share the sweeps, graph replay of the factor and
-sweep launches against the launches issued one by one, and the fall-back
-to block Jacobi where a softened tangent is no longer positive definite."""
+"""GPU parity of the exact preconditioners of models whose band is wide or
+whose equations are many (the tiled sparse factor of xg_tiles.hip) against
+the CPU oracle's direct solve: single solves on a 3D RC frame (half bandwidth
+above 63) and on a quad strip of more than 16,384 equations, a
+DisplacementControl pushover whose two solves per Newton iteration share the
+sweeps, graph replay of the factor and sweep launches against the launches
+issued one by one, and the fall-back to block Jacobi, of the tiled and of the
+one-workgroup band factor, where a softened tangent is no longer positive
+definite."""
 import numpy as np
 import pytest
 
@@ -79,6 +79,7 @@ def test_wide_band_solve_matches_oracle(case):
     assert relerr(Xg, Xo) <= (RTOL if case == "frame3d" else 1e-8)
     bw = c["band_bw"]
     assert bw > (63 if case == "frame3d" else 0), bw
+    assert g.preconditioner() == "tiled"
     assert g.neq > 16384 or bw > 63
     # the exact preconditioner: one or two iterations
     assert c["cg_iters"] - c0["cg_iters"] <= 3 * (c["solves"] - c0["solves"])
@@ -112,7 +113,7 @@ def test_wide_band_pushover_matches_oracle_and_graph_replay():
         assert abs(g.load_factor - o.load_factor) <= RTOL * abs(o.load_factor)
         assert np.array_equal(g.trial_disp(), e.trial_disp()), step
     c = g.counters()
-    assert c["band_bw"] > 63
+    assert c["band_bw"] > 63 and g.preconditioner() == "tiled"
     assert c["cg_iters"] <= 3 * c["solves"]
     for m in models:
         m.close()
@@ -121,7 +122,7 @@ def test_wide_band_pushover_matches_oracle_and_graph_replay():
 def test_wide_band_falls_back_past_the_peak():
     """A DisplacementControl pushover of the 5x5x8 frame through its peak
     (0.25% roof drift per step): where the softened tangent is no longer
-    positive definite the band factor meets a pivot that is not positive and
+    positive definite the tiled factor meets a pivot that is not positive and
     that matrix is solved with block Jacobi instead (counted in
     band_fallbacks); the trajectory stays with the oracle's direct solve to
     1e-9 through and past the peak."""

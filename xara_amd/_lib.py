@@ -92,6 +92,7 @@ SIGNATURES = {
     "get_point_data": (C.c_int, [VP, C.c_int, P_D, P_I]),
     "element_tangent": (C.c_int, [VP, C.c_int, P_D, P_I]),
     "element_resisting_force": (C.c_int, [VP, C.c_int, P_D, P_I]),
+    "preconditioner": (C.c_int, [VP]),
     "get_counters": (C.c_int, [VP, C.POINTER(Counters)]),
     "time_op": (C.c_int, [VP, C.c_int, C.c_int, P_D]),
     "state_size": (C.c_longlong, [VP, C.c_int]),
@@ -116,7 +117,7 @@ SIGNATURES = {
     "material_vjp": (C.c_int, [C.c_int, P_D, P_D, C.c_int, C.c_double, P_D, P_D, P_D, P_D]),
 }
 GPU_ONLY = {k for k in SIGNATURES if k.startswith(("ensemble_", "adjoint_"))} | {
-    "device_name", "material_vjp", "spmv_config", "cg_config", "solve_noalloc"}
+    "device_name", "material_vjp", "spmv_config", "cg_config", "solve_noalloc", "preconditioner"}
 
 
 class Binding:

@@ -727,6 +727,13 @@ int xg_get_counters(xg_domain* h, xg_counters* c) {
   });
 }
 
+int xg_preconditioner(xg_domain* h) {
+  return guard([&] {
+    auto& d = R(h);
+    return d.wide_active() ? XG_PRECOND_TILED : d.band_active() ? XG_PRECOND_BAND : XG_PRECOND_JACOBI;
+  });
+}
+
 int xg_time_op(xg_domain* h, int op, int reps, double* ms) {
   return guard([&] {
     auto& d = R(h);

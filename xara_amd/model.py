@@ -414,6 +414,11 @@ class Model:
         self._check(self._b.get_counters(self._h, C.byref(c)))
         return {k: getattr(c, k) for k, _ in c._fields_}
 
+    def preconditioner(self):
+        """What preconditions the next solve: "jacobi" (blocks or single
+        equations), "band" or "tiled" (an exact factor)."""
+        return ("jacobi", "band", "tiled")[self._check(self._b.preconditioner(self._h))]
+
     def time_op(self, op, reps):
         ms = C.c_double(0)
         self._check(self._b.time_op(self._h, OPS[op], reps, C.byref(ms)))
