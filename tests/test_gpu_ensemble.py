@@ -1,6 +1,6 @@
 """GPU parity of the batched frame ensemble: many independent 2D RC frames of
-uneven size advanced together by Newmark + Newton (one persistent launch per
-Newton iteration, one hipGraph per step) must follow the same trajectories as
+uneven size advanced together by Newmark + Newton (three launches per Newton
+iteration, one hipGraph per step) must follow the same trajectories as
 each frame analysed alone, on the CPU oracle, to 1e-9 relative."""
 import numpy as np
 import pytest
@@ -143,3 +143,54 @@ def test_ensemble_failed_models_stop():
         for k, o in enumerate(orc):
             assert relerr(ens.disp(k), o.trial_disp()) <= RTOL, (step, k)
     assert not all(alive), "no frame failed: the case does not exercise the failure path"
+
+
+# (stories, bays, seed, pga): equations, half bandwidth of the numbering, and
+# the branch of the solve that takes the member
+SOLVES = [(2, 1, 0, 0.5),    # 12, 8: window of 16 rows, more than the equations
+          (7, 1, 1, 0.4),    # 42, 8
+          (5, 3, 3, 0.3),    # 60, 14: window of 32, pivots in batches of 16
+          (4, 4, 2, 0.5),    # 60, 17: window of 32, batches of 8
+          (7, 5, 5, 0.5),    # 126, 20, 22 KB in LDS
+          (6, 6, 4, 0.5),    # 126, 23, 25 KB in LDS
+          (14, 6, 7, 0.4),   # 294, 23, 57.4 KB: the band in memory
+          (20, 6, 6, 0.4),   # 420, 23, 82 KB: in memory
+          (7, 8, 8, 0.5),    # 189, 26: Cholesky by columns, in memory
+          (9, 8, 9, 0.5)]    # 243, 29: the same
+
+
+def band_of(o):
+    rp, ci = o.csr_pattern()
+    return int(np.max(np.abs(np.repeat(np.arange(o.neq), np.diff(rp)) - ci)))
+
+
+def test_ensemble_solves_of_every_kind():
+    """Members on both sides of every limit of the solve: windows of 16 and
+    32 rows, bands in LDS and in memory (where the forward values pass through
+    the solution), bands wider than 24."""
+    print("case: ensemble of 10 frames, 12 to 420 equations", flush=True)
+    ens, _ = make_ensemble(SOLVES)
+    orc = oracles(SOLVES)
+    bw = [band_of(o) for o in orc]
+    lds = [o.neq * (b + 2) * 8 for o, b in zip(orc, bw)]
+    assert min(bw) <= 8 and any(8 < b <= 16 for b in bw) and any(b > 24 for b in bw)
+    assert any(16 < b <= 24 and q <= 56 << 10 for b, q in zip(bw, lds))
+    assert any(b <= 24 and q > 56 << 10 for b, q in zip(bw, lds))
+    for step in range(0, 120, 10):
+        assert ens.analyze(10, DT) == 0, step
+        for k, o in enumerate(orc):
+            assert o.analyze(10, DT) == 0, (step, k)
+            assert relerr(ens.disp(k), o.trial_disp()) <= RTOL, (step, k)
+
+
+def test_ensemble_of_more_than_four_members_to_a_compute_unit():
+    """More than 1,024 members: bands above 38 KB go to memory, which up to
+    there are in LDS; the same arithmetic, so the same bits."""
+    big = (10, 6, 3, 0.5)  # 210 equations, half bandwidth 23: 42 KB
+    print("case: ensemble of 1,030 frames", flush=True)
+    few, _ = make_ensemble([big, (1, 1, 0, 0.3)])
+    many, _ = make_ensemble([(1, 1, 0, 0.3)] * 1029 + [big])
+    for ens in (few, many):
+        assert ens.analyze(60, DT) == 0
+    assert np.array_equal(many.disp(1029), few.disp(0))
+    assert np.array_equal(many.disp(0), few.disp(1)) and np.array_equal(many.disp(1028), few.disp(1))

@@ -4,7 +4,8 @@ gfx950 with the library's flags and reads the assembler's NumVgprs).
 The section update runs latency-bound, so its occupancy matters: the 3D
 kernel sits just under 168 VGPRs (three waves per SIMD; at 169 it drops to
 two and runs about 20% slower), the 2D kernel under 128 (four waves), and
-the ensemble's step kernels are compiled for four waves."""
+the ensemble's kernels (the fiber updates in k_ens_fibers among them) are
+compiled for four waves."""
 import os
 import re
 import shutil
@@ -48,5 +49,5 @@ def test_section_update_register_budget(tmp_path):
 
 def test_ensemble_step_kernels_four_waves(tmp_path):
     res = vgprs(tmp_path, "xg_ensemble.hip")
-    for k in ("k_ens_predictILi256E", "k_ens_iterateILi256E"):
+    for k in ("k_ens_fibersILb0E", "k_ens_fibersILb1E", "k_ens_predictILi256E", "k_ens_iterateILi256E"):
         assert pick(res, k) <= 128
