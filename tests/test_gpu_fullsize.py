@@ -120,7 +120,7 @@ def test_rc_frame_10x10x20_full_size():
     its full size (6,820 elements, 34,100 sections, 4,092,000 fibers, 14,520
     equations): numbering and CSR pattern bit-exact; two
     DisplacementControl steps of the roof (GPU PCG preconditioned by the
-    tiled band factor, half bandwidth 731; the oracle's direct solve) with
+    tiled factor, half bandwidth 731; the oracle's direct solve) with
     the trajectory and load factor to 1e-9; then, from that committed state,
     one update on a lateral field past first cracking: every section's
     deformation, resultant and tangent (the fiber update in rows of 20

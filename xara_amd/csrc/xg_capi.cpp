@@ -603,7 +603,7 @@ int xg_add_a(xg_domain* h, int nblk, int bs, const double* m, const int* id) {
     xg::launch_add_diag(d.stream, (int)pos.size(), dpos.p, dval.p, 1.0, d.vals.p);
     d.sym_stale = true;
     d.pc_done = nullptr;
-    d.wb_failed = false;
+    d.pc_dropped = false;
     XG_HIP(hipStreamSynchronize(d.stream));
     return 0;
   });
@@ -721,7 +721,7 @@ int xg_get_counters(xg_domain* h, xg_counters* c) {
     auto& d = D(h);
     *c = d.counters;
     c->band_bw = d.wide_active() ? d.tl_bw : d.band_active() ? d.band_bw : -1;
-    c->band_fallbacks = d.wb_fallbacks;
+    c->band_fallbacks = d.pc_fallbacks;
     c->band_reuses = d.pc_reuses;
     return 0;
   });

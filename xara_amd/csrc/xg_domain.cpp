@@ -709,7 +709,7 @@ void Domain::setup() {
   if (spmv_format != XG_SPMV_CSR) sym_prepare(true);
   band_order(plan);
   pc_done = nullptr;
-  wb_failed = false;
+  pc_dropped = false;
   XG_HIP(hipStreamSynchronize(s));
   lambda = 0;
   time = 0;
@@ -835,7 +835,7 @@ void Domain::form_tangent() {
   }
   sym_stale = true;
   pc_done = nullptr;
-  wb_failed = false;
+  pc_dropped = false;
   if (tl_formed >= kTileRetry) tl_on = false;
   // Newmark::formNodTangent: c2 C + c3 M of the nodal masses (C = alphaM M)
   if (integ == 3) launch_add_diag(stream, nmass_eq, mass_pos.p, mass_val.p, nm_c3 + nm_c2 * alphaM, vals.p);
@@ -1337,8 +1337,8 @@ int Domain::precond_settle(const CgBufs& w) {
 
 // The exact factor of the current matrix gives way to the PCG without it.
 int Domain::drop_factor() {
-  wb_failed = true;
-  wb_fallbacks++;
+  pc_dropped = true;
+  pc_fallbacks++;
   pc_done = nullptr;
   pc_cache = false;
   return 1;

@@ -251,15 +251,17 @@ struct Domain {
   DVec<double> band2;  // work vectors of a second band solve (solve_pair)
   bool dc_hat_ready = false;  // the Newton iteration has solved for the reference load
   int solve_pair(const double* b1, double* x1, const double* b2, double* x2);
-  bool band_active() const { return cg_small_on && band_bw >= 0 && !wb_failed && !wide_active(); }
+  bool band_active() const { return cg_small_on && band_bw >= 0 && !pc_dropped && !wide_active(); }
   struct TilePlanJob;  // the tiled factor's plan, built on a thread beside the rest of the set-up
   void band_order(TilePlanJob& plan);
   // tiled sparse factorisation (xg_tiles.hip), the exact preconditioner
-  // under the static integrators of the systems tiles_take() accepts (a
-  // transient's K + c3 M is well conditioned by the mass term: block Jacobi
-  // converges in tens of iterations there).  A solve takes one or two PCG
-  // iterations (solve_wide); factor and sweeps are replayed from captured
-  // graphs when cg_graph_on.
+  // under the static integrators of the systems tiles_take() accepts.  A solve
+  // takes one or two PCG iterations (solve_wide); factor and sweeps are
+  // replayed from captured graphs when cg_graph_on.
+  // Not under Newmark: the mass term keeps K + c3 M well conditioned, and block
+  // Jacobi takes 26 to 28 iterations a solve on 3D frames of 576 / 2,160 / 5,832
+  // equations, 0.67 / 1.48 / 1.60 ms a step of about three Newton iterations;
+  // with the factor 0.91 / 1.50 / 2.76.
   // Fewer equations: the one-workgroup band factor (k_band_factor_w), or
   // block Jacobi (k_pcg_small) for bands above 63.  A new matrix and one solve,
   // tiled / without, us: quad strips 120 equations 111 / 98, 256 133 / 149, 360
@@ -291,7 +293,7 @@ struct Domain {
   bool tl_on = false;  // a solve has gone on with the factor
   int tl_formed = 0;   // matrices factored since
   bool tl_big() const { return tl_factor_us > kTileBigUs; }
-  bool tl_usable() const { return cg_small_on && cg_wide_on && !wb_failed && tl_bw >= 0 && integ != 3; }
+  bool tl_usable() const { return cg_small_on && cg_wide_on && !pc_dropped && tl_bw >= 0 && integ != 3; }
   bool tiles_plan(TilePlan& P) const;
   void tiles_plan_start(TilePlanJob& job);
   void tiles_take(TilePlanJob& job);
@@ -319,9 +321,9 @@ struct Domain {
   // positive (an indefinite tangent past a peak), or the PCG failed with the
   // tiled one: its solves fall back to the PCG without it until the next
   // assembly
-  bool wb_failed = false;
-  long long wb_fallbacks = 0;
-  // the values of the matrix whose band factor (either kind) the domain's
+  bool pc_dropped = false;
+  long long pc_fallbacks = 0;
+  // the values of the matrix whose exact factor (band or tiled) the domain's
   // own factor storage holds: a matrix equal to them bit for bit (a model
   // still elastic) keeps its factor instead of being factored again
   // (XG_PC_REUSE=0 turns this off)

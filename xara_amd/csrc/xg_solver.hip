@@ -739,7 +739,7 @@ __global__ __launch_bounds__(256) void k_cg_init_scal(int nb, const double* __re
 // per chunk.  G lanes to a row (G n <= 1,024): each keeps its first K entries
 // in registers for the whole solve, with their columns, reads further ones
 // from memory, and takes p from LDS; K is what the registers of NT threads
-// hold (44 for 768 threads, 24 for 1,024). the row's first lane owns
+// hold (44 for 768 threads, 24 for 1,024).  The row's first lane owns
 // its x, r, p and row of the block inverse.  Sums go through a fixed order
 // of lanes and wavefronts, so every thread holds the same bits and takes the
 // same branches.  The final scalars go to the CGScal the host reads.

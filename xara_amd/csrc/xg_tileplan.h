@@ -9,8 +9,8 @@
 // slightly off them), the separator the nodes of one side that a matrix entry
 // joins to the other.  Both sides are ordered first, the separator last,
 // its nodes by bisection so that a tile holds nodes near each other.  The
-// chain of dependent tile columns is then one branch of separators (34 tile
-// columns on a 10 x 10 x 20 frame) instead of the whole band (227).
+// chain of dependent tile columns is then one branch of separators (37 levels
+// on a 10 x 10 x 20 frame) instead of the whole band (227).
 //
 // Tiles.  Tile column k holds equations at positions 64 k .. 64 k + wid - 1;
 // the rest of its 64 positions are padding.  Its tiles are the diagonal one

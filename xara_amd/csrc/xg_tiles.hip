@@ -20,10 +20,10 @@
 // cores bound (4,096 cycles a tile).  Against a band factor in 64 x 64 tiles
 // with triangular sweeps (one launch per tile column, 41 us each, and two
 // more per column and application): 10 x 10 x 20 frame, 14,520 equations,
-// 227 tile columns there and 37 levels here, two pushover steps 170 -> 38 ms;
-// 150 x 37 quad strip 210 -> 17 ms; 12^3 bricks 42 -> 9.2 ms; a 4 x 3 x 7
-// frame of force-based elements (840 equations, block Jacobi in one
-// workgroup before) 187 -> 6.3 ms.
+// 227 tile columns there and 37 levels here, two pushover steps 170 -> 21 ms;
+// 150 x 37 quad strip, three steps, 210 -> 13.5 ms; 12^3 bricks 42 -> 7.3 ms;
+// a 4 x 3 x 7 frame of force-based elements (840 equations, block Jacobi in
+// one workgroup before) 187 -> 4.5 ms.
 #include <algorithm>
 
 #include "../../include/xara_gpu.h"
