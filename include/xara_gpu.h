@@ -212,10 +212,11 @@ int  xg_spmv_config(xg_domain* d, int format, int lanes);
                           many MiB); without device memory for it the model
                           goes on without it.  The memory is taken at xg_setup
                           for a factor that the first solve uses, else by the
-                          first solve that does.  A factor estimated above 3 ms is first
-                          formed when a solve without it has cost as much,
-                          and used from then on until revertToStart; on by
-                          default                                           */
+                          first solve that does.  A factor estimated
+                          above 2.8 ms is first formed when a solve without
+                          it has cost as much, and used until revertToStart
+                          or until 16 matrices were factored (then the PCG
+                          without it is tried again); on by default          */
 int  xg_cg_config(xg_domain* d, int chunk, int flags);
 /* What preconditions the next solve: XG_PRECOND_JACOBI (nodal blocks or
    single equations), XG_PRECOND_BAND (the one-workgroup band factor) or
