@@ -220,7 +220,8 @@ int  xg_spmv_config(xg_domain* d, int format, int lanes);
 int  xg_cg_config(xg_domain* d, int chunk, int flags);
 /* What preconditions the next solve: XG_PRECOND_JACOBI (nodal blocks or
    single equations), XG_PRECOND_BAND (the one-workgroup band factor) or
-   XG_PRECOND_TILED (XG_CG_WIDE); or a negative error code.                  */
+   XG_PRECOND_TILED (XG_CG_WIDE; not before its memory is taken); or a negative
+   error code.                                                               */
 #define XG_PRECOND_JACOBI 0
 #define XG_PRECOND_BAND   1
 #define XG_PRECOND_TILED  2

@@ -1004,7 +1004,7 @@ bool Domain::tiles_plan(TilePlan& P) const {
 // leaves alone.  Without a thread to spare it runs in tiles_take().
 void Domain::tiles_plan_start(TilePlanJob& job) {
   tl_planned = false;
-  if (num.neq < kTileMinEqn || num.neq > kTileMaxEqn || integ == 3) return;
+  if (num.neq < kTileMinEqn || num.neq > kTileMaxEqn || integ == 3 || !cg_small_on || !cg_wide_on) return;
   auto build = [this, &job] { return tiles_plan(job.plan); };
   try {
     job.done = std::async(std::launch::async, build);
@@ -1031,8 +1031,9 @@ void Domain::tiles_take(TilePlanJob& job) {
   tl_bw = order_bw;
 }
 
-// Before a solve that may allocate: the plan of a model set up for a
-// transient, and the factor's memory, when this solve would take the factor.
+// Before a solve that may allocate: the plan of a model set up as a transient
+// or with the factor off, and the factor's memory, when this solve would take
+// the factor.
 void Domain::tiles_ready() {
   if (!cg_small_on || !cg_wide_on || integ == 3 || tl_mem) return;
   if (!tl_planned) {

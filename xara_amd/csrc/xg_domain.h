@@ -297,8 +297,8 @@ struct Domain {
   bool tiles_plan(TilePlan& P) const;
   void tiles_plan_start(TilePlanJob& job);
   void tiles_take(TilePlanJob& job);
-  // The plan is made at set-up (for a model set up as a transient, at its
-  // first static solve).  The memory, up to 2 x 4 GiB, is taken at set-up
+  // The plan is made at set-up (for a model set up as a transient, or with the
+  // factor off, at its first solve that could use it).  The memory, up to 2 x 4 GiB, is taken at set-up
   // only for a factor that the first solve uses; else by the first solve
   // that does, so that state determination, transients and solids that stay
   // with block Jacobi do without.  The allocation-free solve never takes it.
