@@ -215,8 +215,8 @@ int  xg_spmv_config(xg_domain* d, int format, int lanes);
                           first solve that does.  A factor estimated
                           above 2.8 ms is first formed when a solve without
                           it has cost as much, and used until revertToStart
-                          or until 16 matrices were factored (then the PCG
-                          without it is tried again); on by default          */
+                          or until 64 matrices were factored, when the PCG
+                          without it is tried again; on by default           */
 int  xg_cg_config(xg_domain* d, int chunk, int flags);
 /* What preconditions the next solve: XG_PRECOND_JACOBI (nodal blocks or
    single equations), XG_PRECOND_BAND (the one-workgroup band factor) or

@@ -328,10 +328,9 @@ def test_dropped_factor_keeps_the_warm_start(control, wide):
 
 
 def test_large_solid_tries_block_jacobi_again(monkeypatch):
-    """A solid that has gone on with the factor returns to block Jacobi after
-    16 factored matrices: elastic unloading after plastic steps takes 16
-    factors and then iterations; while the steps stay hard every solve is
-    finished by the factor."""
+    """A solid that has gone on with the factor tries block Jacobi again after
+    64 factored matrices: while the steps stay hard every solve is finished by
+    the factor, elastic unloading returns to iterations at the next try."""
     print("case: large solid 25^3 unloaded", flush=True)
     monkeypatch.setenv("XG_PC_REUSE", "0")  # count a factor for every matrix
     m = Model(3, 3)
@@ -359,11 +358,11 @@ def test_large_solid_tries_block_jacobi_again(monkeypatch):
             its.append(m.counters()["cg_iters"] - c)
             on.append(m.preconditioner() == "tiled")
         return its, on, X
-    its, on, X = solves(1.02, 40)  # loading on: block Jacobi alone would not do
-    assert on == [True] * 40
-    assert 1 <= sum(i > 30 for i in its) <= 3  # the tries
-    its, on, Xe = solves(0.98, 20)
+    its, on, X = solves(1.02, 90)  # loading on: block Jacobi alone would not do
+    assert on == [True] * 90
+    assert 1 <= sum(i > 30 for i in its) <= 2  # the tries
+    its, on, Xe = solves(0.98, 70)
     assert max(its[:1]) <= 3 and on[0] and not on[-1]
-    assert on == sorted(on, reverse=True) and 1 <= sum(on) <= 16
+    assert on == sorted(on, reverse=True) and 1 <= sum(on) <= 64
     assert min(its[sum(on):]) > 30
     m.close()

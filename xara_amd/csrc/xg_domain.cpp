@@ -1390,10 +1390,10 @@ int Domain::solve_with(const double* b, double* x, const CgBufs& w, bool graphs,
     cg_start(stream, n, bs, xs, w.r0, w.z, w.p, bw, sweep ? w.binvs : w.binv, bfirst.p, bsize.p, w.part,
              rtol * rtol, maxit, w.scal, warm ? w.q : nullptr);
     int issued = 0, next = cg_chunk;
-    // whole chunks worth a factor
+    // whole chunks worth a factor and part of the solve with it
     int cap = INT_MAX;
     if (tl_usable() && tl_big() && !tl_on && (own || tl_mem))
-      cap = ((int)(tl_factor_us / tl_iter_us) / cg_chunk + 1) * cg_chunk;
+      cap = ((int)(1.1 * tl_factor_us / tl_iter_us) / cg_chunk + 1) * cg_chunk;
     const int L = lanes();
     while (true) {
       read_status(w);

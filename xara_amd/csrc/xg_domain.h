@@ -281,14 +281,22 @@ struct Domain {
   // 1.05 / 2.17 / 3.93 / 6.64 / 12.6 / 18.6 / 30.3; an iteration from 24^3 on
   // 18.0 / 21.6 / 27.7 / 32.4 / 40.0 us, measured 17.2 / 23.3 / 28.5 / 33.0 /
   // 39.9.  Above kTileBigUs such a model starts with block Jacobi, and a solve
-  // that has not converged after as many iterations as a factor is worth goes
-  // on with the factor: at most about twice the better of the two for that
-  // solve.  The later solves keep the factor until revertToStart, or until
-  // kTileRetry matrices were factored: then block Jacobi is tried again (steps
-  // may have turned mild, 100 to 300 iterations), which costs a sixteenth
-  // where they have not.
+  // that has not converged after as many iterations as a factor and half of its
+  // first solve are worth (1.1 times the factor) goes on with the factor: at
+  // most about twice the better of the two for that solve.  The later solves
+  // keep the factor until revertToStart, or until kTileRetry matrices were
+  // factored: then block Jacobi is tried again (steps may have turned mild, 100
+  // to 300 iterations), for at most one part in kTileRetry where they have not.
+  // Pushovers of J2 blocks to 1.12 times the yield pressure in 2 / 8 / 20 steps,
+  // ms: 24^3 31 / 94 / 189, 28^3 78 / 184 / 345, 33^3 127 / 287 / 637, 38^3 220 /
+  // 607 / 1,018.  With the limit at the factor alone 33^3 133 / 294 / 652 and the
+  // others within 1%, at 1.2 times it 24^3 31.5 / 94 / 190 and 33^3 129 / 277 /
+  // 614, at 1.5 times 28^3 82 / 207 / 375; with 16 in kTileRetry's place another
+  // 2 to 5% at 8 and 20 steps; with the costs taken as 25 us per level, 30 TFLOP/s
+  // and 26 us an iteration, and no return, 28^3 83 / 210 / 349, 33^3 135 / 287 /
+  // 640, 38^3 235 / 667 / 1,040.
   static constexpr double kTileBigUs = 2800.0;
-  static constexpr int kTileRetry = 16;
+  static constexpr int kTileRetry = 64;
   double tl_factor_us = 0, tl_iter_us = 1;
   bool tl_on = false;  // a solve has gone on with the factor
   int tl_formed = 0;   // matrices factored since
